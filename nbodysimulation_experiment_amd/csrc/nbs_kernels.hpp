@@ -157,7 +157,7 @@ void launch_fill_u32(uint32_t *p, uint32_t value, uint64_t n, hipStream_t stream
 // sum rho, max rho, sum |rho - rho0|, sum (rho - rho0)^2, sum x, sum y,
 // non-finite count, finite count, 0) are reduced per workgroup of
 // kDiagPerBlock slots into partials[diagnostics_blocks(n) * kDiagWidth], then
-// combined in workgroup order.
+// combined in a fixed order.
 constexpr int kDiagWidth = 12;
 constexpr int kDiagPerBlock = kBlock * 16;
 void launch_diagnostics(const Buffers &b, const DevParams &p, int n, double *partials, double *out,
