@@ -1119,7 +1119,9 @@ class Simulation {
                RELAX_CALIBRATE = 5, RELAX_SURROGATE_CARRIED = 6 };
 
   struct SurrogateState {
-    DevBuf<float> params, adamM, adamV, grad, out, act, cnt, dH, dG, dM, dO, part, lossPart, loss;
+    DevBuf<float> params, adamM, adamV, grad, out, cnt, part, lossPart, loss;
+    DevBuf<uint4> act;
+    DevBuf<float4> dH;
     DevBuf<uint16_t> w1b, w2b, w3b, w2t, w3t;
     DevBuf<float2> target, shadowX, shadowV, densA, densB, presScratch;
     DevBuf<uint32_t> candScratch, pairPart;
@@ -1192,15 +1194,12 @@ class Simulation {
     if (S.trainCap >= cap_) return;
     const size_t c = cap_;
     S.out.alloc(2 * c);
-    S.act.alloc((size_t)kActStride * c);
+    S.act.alloc((size_t)kActWords * surrogate_tiles(c));
     S.cnt.alloc(c);
-    S.dH.alloc(kHid * c);
-    S.dG.alloc(kHid * c);
-    S.dM.alloc(kHid * c);
-    S.dO.alloc(2 * c);
+    S.dH.alloc((size_t)kGradWords * surrogate_tiles(c));
     S.target.alloc(c);
     S.part.alloc(surrogate_part_floats((int)c));
-    S.lossPart.alloc(2 * (size_t)surrogate_head_blocks((int)c));
+    S.lossPart.alloc(2 * (size_t)surrogate_head_waves((int)c));
     if (S.loss.n < 2) S.loss.alloc(2);
     S.trainCap = c;
   }
@@ -1219,9 +1218,6 @@ class Simulation {
       m.act = S.act.p;
       m.cnt = S.cnt.p;
       m.dH = S.dH.p;
-      m.dG = S.dG.p;
-      m.dM = S.dM.p;
-      m.dO = S.dO.p;
       m.target = S.target.p;
       m.part = S.part.p;
       m.grad = S.grad.p;
@@ -1230,6 +1226,12 @@ class Simulation {
       m.lossIndex = lossIndex;
     }
     return m;
+  }
+  // The next Adam step (betas 0.9 / 0.999, eps 1e-8).
+  AdamStep adamStep(float lr) {
+    SurrogateState &S = *sur_;
+    return {S.params.p, S.adamM.p, S.adamV.p, S.w1b.p, S.w2b.p, S.w3b.p, S.w2t.p, S.w3t.p,
+            lr, 0.9f, 0.999f, 1.0e-8f, (int)++S.adamT};
   }
   // The relaxation phase of a step in the learned modes.
   void enqueueLearnedRelaxation(const DevParams &p, const DevScene &s0, int n, int relax, int lossIndex) {
@@ -1278,10 +1280,8 @@ class Simulation {
         launch_density_error_scenes(S.densA.p, S.densB.p, buf_.keys, buf_.sceneBase, buf_.nScenes, n,
                                     S.sceneErr.p, stream_);
         if (online) {
-          launch_surrogate_backward(buf_, p, s0, n, m, stream_);
-          launch_adam(S.params.p, S.grad.p, S.adamM.p, S.adamV.p, kNumWeights, S.onlineLr, 0.9f, 0.999f, 1.0e-8f,
-                      (int)++S.adamT, stream_);
-          launch_bf16_weights(S.params.p, S.w1b.p, S.w2b.p, S.w3b.p, S.w2t.p, S.w3t.p, stream_);
+          const AdamStep adam = adamStep(S.onlineLr);
+          launch_surrogate_backward(buf_, p, s0, n, m, &adam, stream_);
           ++S.rep.train_steps;
         }
         break;
@@ -1295,12 +1295,12 @@ class Simulation {
         if (relax == RELAX_CALIBRATE) break;
         const SurrogateBufs m = surBufs(true, lossIndex);
         launch_surrogate_forward(buf_, p, s0, n, m, kFwdTrain, stream_);
-        launch_surrogate_backward(buf_, p, s0, n, m, stream_);
         if (relax == RELAX_TRAIN) {
-          launch_adam(S.params.p, S.grad.p, S.adamM.p, S.adamV.p, kNumWeights, S.lr, 0.9f, 0.999f, 1.0e-8f,
-                      (int)++S.adamT, stream_);
-          launch_bf16_weights(S.params.p, S.w1b.p, S.w2b.p, S.w3b.p, S.w2t.p, S.w3t.p, stream_);
+          const AdamStep adam = adamStep(S.lr);
+          launch_surrogate_backward(buf_, p, s0, n, m, &adam, stream_);
           ++S.rep.train_steps;
+        } else {
+          launch_surrogate_backward(buf_, p, s0, n, m, nullptr, stream_);
         }
         break;
       }

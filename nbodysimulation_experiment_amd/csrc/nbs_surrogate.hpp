@@ -46,9 +46,13 @@ constexpr int kNumWeights = kOffB4 + 2;         // trained parameters (9474)
 constexpr int kOffNorm = kNumWeights;
 constexpr int kNumParams = kOffNorm + 8;
 
-constexpr int kActStride = 3 * kHid;            // H, M, G per particle
-constexpr int kSurRows = 32;                    // particles per wave
-constexpr int kOuterRows = 512;                 // particles per outer-product workgroup
+constexpr int kSurRows = 32;                    // particles per MFMA row tile
+// Training activations of one row tile, in 16-byte words laid out as the MFMA
+// operands and results of its 64 lanes (nbs_surrogate.hip): H and M as BF16
+// (4 words a lane each), G as FP32 (8).
+constexpr int kActWords = (4 + 4 + 8) * 64;
+constexpr int kGradWords = 8 * 64;              // dH of one row tile, FP32
+inline size_t surrogate_tiles(size_t n) { return (n + kSurRows - 1) / kSurRows; }
 
 struct SurrogateBufs {
   const float *params;       // kNumParams FP32 (master)
@@ -57,13 +61,13 @@ struct SurrogateBufs {
   const uint16_t *w3b;       // 64 x 64 BF16
   const uint16_t *w2t, *w3t; // transposes of W2, W3 (BF16), for the backward pass
   float *out;                // N x 2 network output o (may be null)
-  float *act;                // N x 192: H, M, G (training)
+  uint4 *act;                // kActWords per row tile: H, M, G (training)
   float *cnt;                // N: pairs per particle (training)
-  float *dH, *dG, *dM, *dO;  // N x 64, 64, 64, 2 (training)
+  float4 *dH;                // kGradWords per row tile: the loss's gradient with respect to H (training)
   const float2 *target;      // N: plain relaxation displacement (training)
   float *part;               // partial sums of the weight gradient
   float *grad;               // kNumWeights
-  float *lossPart;           // per head workgroup: squared error, squared target
+  float *lossPart;           // per wave of the head's backward pass: squared error, squared target
   float *loss;               // two values per training step at 2 * lossIndex:
                              // mean squared error, relative error
   int lossIndex;
@@ -78,19 +82,25 @@ constexpr int kFwdTrain = 2;
 constexpr int kFwdPressure = 4;  // with kFwdState: also pres = (k (rho - rho0), k_near rho_near) from b.dens
 void launch_surrogate_forward(const Buffers &b, const DevParams &p, const DevScene &s0, int n,
                               const SurrogateBufs &m, int mode, hipStream_t stream);
+// One Adam step on the master weights, and their BF16 copies.
+struct AdamStep {
+  float *params, *m, *v;
+  uint16_t *w1b, *w2b, *w3b, *w2t, *w3t;
+  float lr, b1, b2, eps;
+  int t;  // 1 for the first step
+};
 // Gradient of L for the frame of the last training forward into m.grad
-// (overwritten) and the losses into m.loss[2 * m.lossIndex ...].
+// (overwritten) and the losses into m.loss[2 * m.lossIndex ...]; with adam set,
+// then one step on the weights.
 void launch_surrogate_backward(const Buffers &b, const DevParams &p, const DevScene &s0, int n,
-                               const SurrogateBufs &m, hipStream_t stream);
+                               const SurrogateBufs &m, const AdamStep *adam, hipStream_t stream);
 // Workgroups of the forward pass (one pair count each) for n particles.
 int surrogate_forward_waves(int n);
 // Sizes of the partial-sum buffer (floats) and of lossPart (pairs) for n particles.
 size_t surrogate_part_floats(int n);
-int surrogate_head_blocks(int n);
+int surrogate_head_waves(int n);
 void launch_bf16_weights(const float *params, uint16_t *w1b, uint16_t *w2b, uint16_t *w3b, uint16_t *w2t,
                          uint16_t *w3t, hipStream_t stream);
-void launch_adam(float *params, const float *grad, float *m, float *v, int count, float lr, float b1, float b2,
-                 float eps, int t, hipStream_t stream);
 // out[0] = sum |a.x - b.x|, out[1] = sum b.x over n (FP64), partials sized
 // diagnostics_blocks(n) x 2.
 void launch_density_error(const float2 *a, const float2 *b, int n, double *partials, double *out,
