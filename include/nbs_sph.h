@@ -207,7 +207,7 @@ nbs_status nbs_set_options(nbs_sim *sim, uint32_t flags);
  * read neighbours from HBM/L2).  With autotune on, the library times every capacity on real steps
  * (all capacities give bit-identical results) and keeps the fastest per
  * kernel, again every retune_interval steps (0: once; default 256); steps of
- * fewer than 1,024 particles use the wide kernels.  No reference
+ * at most 65,536 particles use the wide kernels.  No reference
  * counterpart: the reference's only tunable is its thread count. */
 typedef struct nbs_tuning {
   int32_t autotune;          /* 0: tile_cap fixed; 1: tune now, then every retune_interval steps;
@@ -215,7 +215,7 @@ typedef struct nbs_tuning {
                                    nbs_get_tuning then reports 1) */
   uint32_t retune_interval;
   int32_t tile_cap[3]; /* viscosity, density, relaxation: LDS tile capacity 0, 1024, 2048 or 4096, or
-                          -1 for the wide kernels (one wave per particle); all give identical results */
+                          -1 for the wide kernels (several lanes per particle); all give identical results */
   int32_t wide_max_particles; /* steps with at most this many particles use the wide kernels for all three
                                  phases whatever tile_cap says; 0 (default) leaves the choice to tile_cap */
 } nbs_tuning;

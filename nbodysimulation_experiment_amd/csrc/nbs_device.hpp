@@ -105,6 +105,29 @@ __device__ __forceinline__ void pair_length(float r2, float &r, float &inv) {
   inv = rcp_near(r);
 }
 
+// The same results for r2 == 0 or r2 >= 2^-96 (wave_near checks this once per
+// wave), from one v_rsq_f32: y = rsq(x), s0 = x*y, r = s0 + (x - s0^2) * y/2,
+// which is the correctly rounded root for every mantissa, and the reciprocal's
+// Newton step from v_rcp_f32(r) (starting it from y misses the two operands
+// whose root has an all-ones mantissa).  x = r2 + 2^-126 is r2 unless r2 == 0,
+// whose r is then 2^-63: 1 - r/h still rounds to 1 for h > 2^-36, and a zero
+// difference times the finite inv is the zero normal.  9 issue cycles against
+// pair_length's 14, 24 with its form for tiny operands, which every wave with a
+// particle's pair with itself takes (measured rates: FP32 add/mul/FMA 0.7,
+// compares and selects 1.1, transcendentals 2.0 of a CU cycle).
+__device__ __forceinline__ float near_sqrt(float r2) {
+  const float x = r2 + 0x1p-126f;
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float s0 = x * y, h = 0.5f * y;
+  const float d = __builtin_fmaf(-s0, s0, x);
+  return __builtin_fmaf(d, h, s0);
+}
+
+__device__ __forceinline__ void near_length(float r2, float &r, float &inv) {
+  r = near_sqrt(r2);
+  inv = rcp_near(r);
+}
+
 // ---------------------------------------------------------------------------
 // Boundary collisions (sph.h:514-681), bodies of the scene in insertion order
 // (demo4.cpp:414-441).

@@ -2,12 +2,13 @@
 //
 // One step is five kernel groups on one stream:
 //   1. k_visc_predict   integrate, viscosity (Jacobi gather over the previous
-//                       binning), predict, cell key of the predicted position and
-//                       the per-cell arrival count (demo4.cpp:301-356)
-//   2. k_scan_reduce + k_scan_final (k_scan_small for small grids)
+//                       binning), predict, cell key of the predicted position
+//                       (demo4.cpp:301-356)
+//   2. k_count_fill     per-cell arrival count (large steps: within 1)
+//      k_scan_reduce + k_scan_final (k_scan_small for small grids)
 //                       exclusive scan of the per-cell counts -> cell starts
-//   3. k_place (grids above kSmallGridCells cells once every particle is
-//      binned), else k_scatter + k_rank_reorder
+//   3. k_place (large steps once every particle is binned), else k_scatter +
+//      k_rank_reorder
 //                       bucket the particles by cell, order each cell by the
 //                       particles' previous slots (a stable counting sort of the
 //                       slot order), and move the state into the new slot order
@@ -15,15 +16,15 @@
 //   5. k_delta          double-density relaxation (Jacobi gather), plane /
 //                       circle / segment / polygon collisions, velocity
 //                       (demo4.cpp:239-255, 411-450)
-// Small steps use the wide variants of 1, 4 and 5 (one wave per particle;
-// 1 is then followed by k_count_fill, or for the smallest steps the counting
-// and the bucketing move into the one-workgroup scan, k_count_scan_small,
-// whose records k_rank_reorder reads).
+// Small steps use the wide variants of 1, 4 and 5 (several lanes per particle),
+// and for the smallest the counting, the scan and the bucketing are one
+// workgroup's, k_count_scan_small, whose records k_rank_reorder reads.
 //
 // Every FP32 expression keeps the reference's operand order and the library
 // is compiled with -ffp-contract=off and correctly rounded sqrt / divide, so the
 // arithmetic of each pair term is the reference's (sph.h:465-542).
 #include <algorithm>
+#include <type_traits>
 
 #include "nbs_device.hpp"
 
@@ -117,133 +118,112 @@ __device__ __forceinline__ uint32_t for_each_pair(const uint32_t *start, const D
   return cand;
 }
 
-// Wide pair walk for small particle counts: one wave per particle.  Lane t
-// tests candidate base + t of a 64-candidate chunk and, when the pair is in
-// range, term(j, Rx, Ry, r2, G[j], t) computes the pair's K terms and says
-// whether it contributes.  The contributions are then applied in candidate
-// order to two accumulators held in lanes 0 and 1: for each contributing pair
-// and each of STAGES stages s, lane c in {0, 1} does acc -= t[(2s + c) % K]
-// (SUB) or acc += t[(2s + c) % K], reading the terms back from the wave's LDS
-// rows (lds: 65 * K floats; row 64 holds the neutral value +0 for SUB, -0
-// otherwise, which leaves an accumulator unchanged bit for bit and pads groups
-// of four pairs).  So the accumulation performs the same FP32 operations in
-// the same order as the one-lane-per-particle walk; only the per-pair
-// arithmetic runs in parallel across the wave.  acc0 and acc1 are the
-// accumulators' initial and final values (the same in every lane).
-// The chunks are the 64-candidate pieces of the rows dy = -1, 0, 1 in order;
-// the row ranges are the wave's particle's, so the chunk sequence is
-// wave-uniform.  The position (and G value) loads of the first kWideAhead
-// chunks are issued together before the first is used (a particle of a
-// crowded scene has several chunks, and one chunk ahead left a memory latency
-// per chunk on the wave's path); later chunks are loaded one ahead.  idx(1, .)
-// of the particle's own row, which always holds the particle, serves as the
-// in-range address of the lanes past a row's end.  Returns the candidate count.
-constexpr uint32_t kWideAhead = 8;
+// Wide pair walk for small particle counts: G lanes per particle (16, a DPP
+// row, or 4, a quad), so 64 / G particles per wave.  The group tests G
+// candidates at a time (consecutive slots: one coalesced load of positions and
+// of their values G, four chunks in flight) and appends the pairs in range, in
+// candidate order, to its list in LDS (ranks from the wave's ballot).  Then its
+// lanes take G listed pairs at a time: each computes one pair's terms, and the
+// terms are applied in candidate order by broadcasting lane 0, 1, ... of the
+// group (one DPP subtraction or addition each, no LDS), every lane keeping the
+// same sums.  So the accumulation performs the same FP32 operations in the same
+// order as the one-lane-per-particle walk.
+// keep(Rx, Ry, r2, value of j, entry) makes a list entry and says whether the
+// pair may contribute; use(entry, in, left) computes the lane's terms (neutral
+// when !in) and applies those of the batch's first `left` lanes.  Four chunks
+// are tested and listed without a branch between them: with a branch and a
+// list check per chunk the one wave per SIMD of a 4,096-particle step waited
+// for its own scalar unit.
+// The chunks are those of the rows dy = -1, 0, 1 in order; the particle's own
+// slot serves as the in-range address of lanes past a row's end.  Returns the
+// candidate count.
+constexpr int kGroupList = 8;  // list entries per lane of the group
 
-template <int K, int STAGES, bool SUB, typename Idx, typename Term>
+template <int G>
+__device__ __forceinline__ uint32_t group_bits(uint64_t m) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t half = lane < 32u ? (uint32_t)m : (uint32_t)(m >> 32);
+  return (half >> (lane & 31u & ~(uint32_t)(G - 1))) & ((1u << G) - 1u);
+}
+
+// Value v of lane T of the group, in all its lanes.
+template <int G, int T>
+__device__ __forceinline__ float group_lane(float v) {
+  static_assert(G == 16 || G == 4, "a DPP row or quad");
+  constexpr int kCtrl = G == 16 ? 0x150 + T /* row_newbcast */ : T * 0x55 /* quad_perm T,T,T,T */;
+  const int i = __float_as_int(v);
+  return __int_as_float(__builtin_amdgcn_update_dpp(i, i, kCtrl, 0xF, 0xF, true));
+}
+
+// f<0>(), f<1>(), ... f<G - 1>() in order, in blocks of four of which those at
+// or past `left` (wave-uniform) are skipped.
+template <int G, typename F, int T = 0>
+__device__ __forceinline__ void group_apply(int left, F &&f) {
+  if constexpr (T < G) {
+    if (T > 0 && left <= T) return;
+    f(std::integral_constant<int, T>());
+    f(std::integral_constant<int, T + 1>());
+    f(std::integral_constant<int, T + 2>());
+    f(std::integral_constant<int, T + 3>());
+    group_apply<G, F, T + 4>(left, static_cast<F &&>(f));
+  }
+}
+
+template <int G, bool VALUES, typename Entry, typename Keep, typename Use>
 __device__ __forceinline__ uint32_t for_each_pair_wide(const uint32_t *start, const DevScene &sc, int cx, int cy,
-                                                       const float2 *X, Idx idx, float2 xi, float h2, const float2 *G,
-                                                       float *lds, float &acc0, float &acc1, Term &&term) {
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t c = lane & 1u;
-  if (lane < (uint32_t)K) lds[64 * K + lane] = SUB ? 0.0f : -0.0f;
-  float acc = c ? acc1 : acc0;
+                                                       const float2 *X, const float2 *V, uint32_t own, float2 xi,
+                                                       float h2, Entry *list, Keep &&keep, Use &&use) {
+  constexpr uint32_t kCap = kGroupList * G, kAhead = 4;
+  const uint32_t sub = threadIdx.x & (uint32_t)(G - 1), below = (1u << sub) - 1u;
   RowRange rr[3];
   row_ranges(start, sc, cx, cy, rr);
-  uint32_t j0[3], j1[3], nc[3];
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {  // wave-uniform
-    j0[d] = (uint32_t)__builtin_amdgcn_readfirstlane((int)rr[d].j0);
-    j1[d] = (uint32_t)__builtin_amdgcn_readfirstlane((int)rr[d].j1);
-    nc[d] = (j1[d] - j0[d] + 63u) / 64u;
-  }
-  const uint32_t cand = (j1[0] - j0[0]) + (j1[1] - j0[1]) + (j1[2] - j0[2]);
-  const uint32_t nch = nc[0] + nc[1] + nc[2];
-  const uint32_t own = idx(1, j0[1]);  // an in-range slot (the own row holds the particle)
-  // chunk k: row d, first slot base, row end
-  auto chunk = [&](uint32_t k, int &d, uint32_t &base, uint32_t &end) {
-    if (k < nc[0]) {
-      d = 0;
-      base = j0[0] + 64u * k;
-    } else if (k < nc[0] + nc[1]) {
-      d = 1;
-      base = j0[1] + 64u * (k - nc[0]);
-    } else {
-      d = 2;
-      base = j0[2] + 64u * (k - nc[0] - nc[1]);
-    }
-    end = j1[d];
-  };
-  auto load = [&](uint32_t k, float2 &x, float2 &g, bool &in, uint32_t &j) {
-    int d;
-    uint32_t base, end;
-    chunk(k, d, base, end);
-    j = base + lane;
-    in = j < end;
-    x = X[in ? idx(d, base) + lane : own];
-    if (G) g = G[in ? j : own];
-  };
-  auto process = [&](float2 xj, float2 gj, bool in, uint32_t j) {
-    float t[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) t[k] = 0.0f;
-    bool ok = false;
-    if (in) {
-      const float Rx = xj.x - xi.x, Ry = xj.y - xi.y;
-      const float r2 = Rx * Rx + Ry * Ry;
-      if (r2 < h2) ok = term(j, Rx, Ry, r2, gj, t);
-    }
-#pragma unroll
-    for (int k = 0; k < K; ++k) lds[lane * K + k] = t[k];
-    uint64_t mask = __ballot(ok);
-    while (mask) {
-      uint32_t q[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        q[u] = mask ? (uint32_t)__builtin_ctzll(mask) : 64u;
-        mask &= mask - 1u;  // no-op once empty
+  const uint32_t l0 = rr[0].j1 - rr[0].j0, l1 = rr[1].j1 - rr[1].j0, l2 = rr[2].j1 - rr[2].j0;
+  const uint32_t c0 = (l0 + G - 1u) / G, c1 = c0 + (l1 + G - 1u) / G, chunks = c1 + (l2 + G - 1u) / G;
+  // first slot of chunk k of row d: base + k * G
+  const uint32_t b0 = rr[0].j0 + sub, b1 = rr[1].j0 - c0 * G + sub, b2 = rr[2].j0 - c1 * G + sub;
+  uint32_t cnt = 0;
+  if (sub == 0u) list[0] = Entry{};  // read by the lanes past a group's end, also when it never has a pair
+  for (uint32_t k0 = 0;; k0 += kAhead) {
+    const bool done = __ballot(k0 < chunks) == 0ull;  // wave-uniform
+    if (done || __ballot(cnt > kCap - kAhead * G)) {
+      for (uint32_t q = 0; __ballot(q < cnt); q += G) {
+        const bool in = q + sub < cnt;
+        // the entries past the middle of the batch: applied only when some group has them
+        const bool half = G == 16 && __ballot(q + 8u < cnt) == 0ull;
+        use(list[in ? q + sub : 0u], in, half ? G / 2 : G);
       }
-      float v[4][STAGES];
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int st = 0; st < STAGES; ++st) v[u][st] = lds[q[u] * K + (2 * st + c) % K];
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int st = 0; st < STAGES; ++st) acc = SUB ? acc - v[u][st] : acc + v[u][st];
+      cnt = 0u;
+      if (done) break;
     }
-  };
-  float2 xa[kWideAhead], ga[kWideAhead];
-  bool ia[kWideAhead];
-  uint32_t ja[kWideAhead];
+    float2 x[kAhead], v[kAhead];
+    bool in[kAhead];
 #pragma unroll
-  for (uint32_t k = 0; k < kWideAhead; ++k) {
-    if (k >= nch) break;  // wave-uniform
-    ga[k] = make_float2(0.0f, 0.0f);
-    load(k, xa[k], ga[k], ia[k], ja[k]);
-  }
+    for (uint32_t u = 0; u < kAhead; ++u) {
+      const uint32_t k = k0 + u;
+      const uint32_t j = (k < c0 ? b0 : (k < c1 ? b1 : b2)) + k * G;
+      in[u] = j < (k < c0 ? rr[0].j1 : (k < c1 ? rr[1].j1 : rr[2].j1)) && k < chunks;
+      const uint32_t at = in[u] ? j : own;
+      x[u] = X[at];
+      v[u] = VALUES ? V[at] : make_float2(0.0f, 0.0f);
+    }
+    bool hit[kAhead];
+    uint64_t m[kAhead];
+    Entry e[kAhead];
 #pragma unroll
-  for (uint32_t k = 0; k < kWideAhead; ++k) {
-    if (k >= nch) break;
-    process(xa[k], ga[k], ia[k], ja[k]);
-  }
-  if (nch > kWideAhead) {  // the rest, one chunk ahead
-    float2 xn, gn = make_float2(0.0f, 0.0f);
-    bool inN;
-    uint32_t jn;
-    load(kWideAhead, xn, gn, inN, jn);
-    for (uint32_t k = kWideAhead; k < nch; ++k) {
-      const float2 xj = xn, gj = gn;
-      const bool in = inN;
-      const uint32_t j = jn;
-      if (k + 1u < nch) load(k + 1u, xn, gn, inN, jn);
-      process(xj, gj, in, j);
+    for (uint32_t u = 0; u < kAhead; ++u) {
+      const float Rx = x[u].x - xi.x, Ry = x[u].y - xi.y;
+      const float r2 = Rx * Rx + Ry * Ry;
+      hit[u] = keep(Rx, Ry, r2, v[u], e[u]) && in[u] && r2 < h2;
+      m[u] = __ballot(hit[u]);
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kAhead; ++u) {
+      const uint32_t bits = group_bits<G>(m[u]);
+      if (hit[u]) list[cnt + (uint32_t)__popc(bits & below)] = e[u];
+      cnt += (uint32_t)__popc(bits);
     }
   }
-  acc0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 0));
-  acc1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), 1));
-  return cand;
+  return l0 + l1 + l2;
 }
 
 // Arrival index of this lane's particle in cell `key`: lanes of the wave with
@@ -273,6 +253,20 @@ __device__ __forceinline__ uint32_t wave_aggregated_fill(uint32_t *count, uint32
   return base + rank;
 }
 
+// Whether near_length serves this wave's active lanes: h > 2^-36, and no
+// particle with |x| or |y| below 2^-23 (two different floats of which one is
+// 2^-23 or more differ by 2^-47 or more, so every pair of such a particle has
+// r2 == 0 or r2 >= 2^-96).
+__device__ __forceinline__ bool wave_near(const DevParams &p, float2 x) {
+  return p.h > 0x1p-36f && __ballot(fminf(fabsf(x.x), fabsf(x.y)) < 0x1p-23f) == 0ull;
+}
+__device__ __forceinline__ void length_of(bool near, float r2, float &r, float &inv) {
+  if (near)  // wave-uniform
+    near_length(r2, r, inv);
+  else
+    pair_length(r2, r, inv);
+}
+
 // Appends `value` of every lane with `flag` to list[*counter ...] with one
 // atomic per wave; entries at cap or beyond are dropped.  All active lanes must
 // call it.
@@ -290,6 +284,20 @@ __device__ __forceinline__ void wave_append(uint32_t *list, uint32_t *counter, u
 }
 
 constexpr uint32_t kFarFlag = 0x80000000u;  // bit 31 of keyp in placement mode
+
+// Writes the new cell of particle i.  In placement mode it is also counted
+// (k_place orders the cells), and a particle that left the 3x3 cells around
+// its last cell (far) is flagged and listed; otherwise a later kernel counts.
+// All active lanes must call it.
+__device__ __forceinline__ void put_key(const Buffers &b, uint32_t key, bool far, int i, int n) {
+  if (b.farList) {
+    b.keyp[i] = key | (far ? kFarFlag : 0u);
+    (void)wave_aggregated_fill(b.count, key);
+    wave_append(b.farList, b.farCount, (uint32_t)n, far, (uint32_t)i);
+  } else {
+    b.keyp[i] = key;
+  }
+}
 
 // ---------------------------------------------------------------------------
 // 1. integrate + viscosity + predict + key + count
@@ -387,17 +395,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_predict(Buffers b, DevParams p,
   const int cx = cell_coord(xpx, sc.halfW, sc.cellSize, sc.nx);
   const int cy = cell_coord(xpy, sc.halfH, sc.cellSize, sc.ny);
   const uint32_t key = sc.cellBase + (uint32_t)(cy * sc.nx + cx);
-  if (b.farList) {
-    // placement mode: counts only (k_place orders the cells); a particle that
-    // left the 3x3 cells around its last cell is flagged and listed
-    const bool far = abs(cx - pcx) > 1 || abs(cy - pcy) > 1;
-    b.keyp[i] = key | (far ? kFarFlag : 0u);
-    (void)wave_aggregated_fill(b.count, key);
-    wave_append(b.farList, b.farCount, (uint32_t)n, far, (uint32_t)i);
-  } else {
-    b.keyp[i] = key;
-    b.fill[i] = wave_aggregated_fill(b.count, key);
-  }
+  put_key(b, key, abs(cx - pcx) > 1 || abs(cy - pcy) > 1, i, n);
 }
 
 // Restores the per-slot scene and zero acceleration of particles that lose
@@ -1130,20 +1128,21 @@ __global__ __launch_bounds__(kBlock) void k_delta(Buffers b, DevParams p, DevSce
 }
 
 // ---------------------------------------------------------------------------
-// Wide variants for small particle counts: one wave per particle, the pair
-// terms computed across the wave and accumulated in candidate order
+// Wide variants for small particle counts: G lanes per particle, the pair
+// terms computed across them and accumulated in candidate order
 // (for_each_pair_wide), so results equal the one-lane-per-particle kernels'
-// bit for bit.  Used when a step has at most nbs_tuning.wide_max_particles
-// particles: there, one lane per particle leaves most of the chip idle and
+// bit for bit.  There, one lane per particle leaves most of the chip idle and
 // each particle's serial candidate walk sets the kernel time.
 // ---------------------------------------------------------------------------
-constexpr int kWidePerBlock = kBlock / 64;
+template <int G>
+constexpr int kWidePer = kBlock / G;  // particles per workgroup
 
-template <bool MULTI>
+template <bool MULTI, int G>
 __global__ __launch_bounds__(kBlock) void k_visc_predict_wide(Buffers b, DevParams p, DevScene s0, int n, int nBinned,
                                                               int lists) {
-  const int i = (int)(blockIdx.x * kWidePerBlock + (threadIdx.x >> 6));
-  if (i >= n) return;  // whole wave
+  __shared__ float4 list[kBlock * kGroupList];
+  const int group = (int)threadIdx.x / G;
+  const int at = (int)(blockIdx.x * kWidePer<G>) + group, i = min(at, n - 1);  // groups past n repeat the last
   const float2 xi = b.x0[i];
   const float2 vi = b.v[i];
   const bool binned = i < nBinned;
@@ -1161,99 +1160,112 @@ __global__ __launch_bounds__(kBlock) void k_visc_predict_wide(Buffers b, DevPara
   }
   float vx = (aX * p.dt) + vi.x;                         // demo4.cpp:307
   float vy = (aY * p.dt) + vi.y;
+  int pcx = -2, pcy = -2;  // cell of the last binning (none: not adjacent to any cell)
   if (lists && binned) {
     const uint32_t local = b.keys[i] - sc.cellBase;
-    const int cy = (int)(local / (uint32_t)sc.nx);
-    const int cx = (int)local - cy * sc.nx;
-    __shared__ float lds[kWidePerBlock][65 * 2];
+    pcy = (int)(local / (uint32_t)sc.nx);
+    pcx = (int)local - pcy * sc.nx;
     float accx = 0.0f, accy = 0.0f;
-    // per pair: accx -= ix, accy -= iy (own visit), then again (neighbour's visit)
-    for_each_pair_wide<2, 2, true>(
-        b.startCur, sc, cx, cy, b.x0, SlotIndex(), xi, p.h2, b.v, lds[threadIdx.x >> 6], accx, accy,
-        [&](uint32_t, float Rx, float Ry, float r2, float2 vj, float *t) {
-          const float vjx = p.gdtx + vj.x, vjy = p.gdty + vj.y;
+    const bool near = wave_near(p, xi);
+    for_each_pair_wide<G, true>(
+        b.startCur, sc, pcx, pcy, b.x0, b.v, (uint32_t)i, xi, p.h2, list + group * (kGroupList * G),
+        [&](float Rx, float Ry, float, float2 vj, float4 &e) {
+          e = make_float4(Rx, Ry, p.gdtx + vj.x, p.gdty + vj.y);
+          // u > 0 (below) needs (v_i - v_j) . R > 0 up to rounding: pairs that
+          // separate are not listed (half of them)
+          const float a = (vx - e.z) * Rx, c = (vy - e.w) * Ry;
+          return !(a + c < -0x1p-16f * (fabsf(a) + fabsf(c)));
+        },
+        [&](float4 e, bool in, int left) {
+          const float r2 = e.x * e.x + e.y * e.y;
           float r, inv;
-          pair_length(r2, r, inv);                              // sph.h:503, 505
+          length_of(near, r2, r, inv);                          // sph.h:503, 505
           const float qq = r * p.invH;                          // sph.h:504
-          const float nX = Rx * inv, nY = Ry * inv;
-          const float u = (vx - vjx) * nX + (vy - vjy) * nY;    // sph.h:506
-          if (!(u > 0.0f)) return false;
-          const float f = (1.0f - qq) * (p.sigma * u + p.beta * (u * u));  // sph.h:508
-          t[0] = ((f * nX) * 0.5f) * p.dt;                      // demo4.cpp:233
-          t[1] = ((f * nY) * 0.5f) * p.dt;
-          return true;
+          const float nX = e.x * inv, nY = e.y * inv;
+          const float u = (vx - e.z) * nX + (vy - e.w) * nY;    // sph.h:506
+          const float f = (in && u > 0.0f) ? (1.0f - qq) * (p.sigma * u + p.beta * (u * u)) : 0.0f;  // sph.h:507-508
+          const float ix = ((f * nX) * 0.5f) * p.dt;            // demo4.cpp:233
+          const float iy = ((f * nY) * 0.5f) * p.dt;
+          group_apply<G>(left, [&](auto t) {
+            const float bx = group_lane<G, decltype(t)::value>(ix), by = group_lane<G, decltype(t)::value>(iy);
+            accx = accx - bx;                                   // own visit
+            accy = accy - by;
+            accx = accx - bx;                                   // neighbour's visit
+            accy = accy - by;
+          });
         });
     vx = accx + vx;
     vy = accy + vy;
   }
-  if ((threadIdx.x & 63) == 0) {
-    const float xpx = (vx * p.dt) + xi.x;                // demo4.cpp:334-335
-    const float xpy = (vy * p.dt) + xi.y;
-    b.xp[i] = make_float2(xpx, xpy);
-    const int cx = cell_coord(xpx, sc.halfW, sc.cellSize, sc.nx);
-    const int cy = cell_coord(xpy, sc.halfH, sc.cellSize, sc.ny);
-    const uint32_t key = sc.cellBase + (uint32_t)(cy * sc.nx + cx);
-    b.keyp[i] = key;  // counted by k_count_fill
-  }
+  if ((threadIdx.x & (G - 1)) != 0 || at >= n) return;
+  const float xpx = (vx * p.dt) + xi.x;                  // demo4.cpp:334-335
+  const float xpy = (vy * p.dt) + xi.y;
+  b.xp[i] = make_float2(xpx, xpy);
+  const int cx = cell_coord(xpx, sc.halfW, sc.cellSize, sc.nx);
+  const int cy = cell_coord(xpy, sc.halfH, sc.cellSize, sc.ny);
+  const uint32_t key = sc.cellBase + (uint32_t)(cy * sc.nx + cx);
+  put_key(b, key, abs(cx - pcx) > 1 || abs(cy - pcy) > 1, i, n);
 }
 
-// Cell counting after the wide viscosity kernel: one lane per particle, so
-// particles of one cell share wave-aggregated atomics instead of one atomic
-// per particle on the same counter.
+// Cell counting of a step that does not place: one lane per particle in slot
+// order, lanes of a wave with the same cell sharing an atomic.  A kernel of its
+// own, because it runs through the slots in order: particles then arrive in
+// their buckets nearly in slot order, and the rank pass, which moves the
+// particles from bucket order, reads them nearly in sequence.  Counted by the
+// viscosity kernels' waves as they ended, the collapsed 32,400-particle block's
+// grid phase took 39 us, with this launch 22.
 __global__ __launch_bounds__(kBlock) void k_count_fill(Buffers b, int n) {
   const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
   if (i >= n) return;
   b.fill[i] = wave_aggregated_fill(b.count, b.keyp[i]);  // arrival slot; the rank pass orders the cell
 }
 
-// Candidate-count statistics: one min/max pair per workgroup (kWidePerBlock
-// particles), slot blockIdx.x.
-template <bool MULTI>
+// Candidate-count statistics: one min/max pair per workgroup, slot blockIdx.x.
+template <bool MULTI, int G>
 __global__ __launch_bounds__(kBlock) void k_density_wide(Buffers b, DevParams p, DevScene s0, int n) {
-  __shared__ uint32_t shCand[kWidePerBlock];
-  __shared__ float lds[kWidePerBlock][65 * 2];
-  const int w = (int)(threadIdx.x >> 6);
-  const int i = (int)(blockIdx.x * kWidePerBlock + w);
-  if (i < n) {  // whole wave
-    const uint32_t key = b.keys[i];
-    const DevScene sc = scene_of_slot<MULTI>(b, s0, key);
-    const uint32_t local = key - sc.cellBase;
-    const int cy = (int)(local / (uint32_t)sc.nx);
-    const int cx = (int)local - cy * sc.nx;
-    const float2 xi = b.x1[i];
-    float d0 = 0.0f, d1 = 0.0f;
-    // per pair: d0 += term^2, d1 += term^3 (sph.h:473-474)
-    const uint32_t cand = for_each_pair_wide<2, 1, false>(
-        b.startNext, sc, cx, cy, b.x1, SlotIndex(), xi, p.h2, nullptr, lds[w], d0, d1,
-        [&](uint32_t, float, float, float r2, float2, float *t) {
-          const float r = pair_sqrt(r2);                        // sph.h:471
-          const float term = 1.0f - r * p.invH;                 // sph.h:472
-          t[0] = term * term;
-          t[1] = (term * term) * term;
-          return true;
+  __shared__ float list[kBlock * kGroupList];
+  const int group = (int)threadIdx.x / G;
+  const int at = (int)(blockIdx.x * kWidePer<G>) + group, i = min(at, n - 1);
+  const uint32_t key = b.keys[i];
+  const DevScene sc = scene_of_slot<MULTI>(b, s0, key);
+  const uint32_t local = key - sc.cellBase;
+  const int cy = (int)(local / (uint32_t)sc.nx);
+  const int cx = (int)local - cy * sc.nx;
+  const float2 xi = b.x1[i];
+  float d0 = 0.0f, d1 = 0.0f;
+  const bool near = wave_near(p, xi);
+  const uint32_t cand = for_each_pair_wide<G, false>(
+      b.startNext, sc, cx, cy, b.x1, nullptr, (uint32_t)i, xi, p.h2, list + group * (kGroupList * G),
+      [&](float, float, float r2, float2, float &e) {
+        e = r2;
+        return true;
+      },
+      [&](float r2, bool in, int left) {
+        const float r = near ? near_sqrt(r2) : pair_sqrt(r2);   // sph.h:471
+        const float term = in ? 1.0f - r * p.invH : 0.0f;       // sph.h:472
+        const float t2 = term * term, t3 = (term * term) * term;
+        group_apply<G>(left, [&](auto t) {
+          d0 = d0 + group_lane<G, decltype(t)::value>(t2);      // sph.h:473
+          d1 = d1 + group_lane<G, decltype(t)::value>(t3);      // sph.h:474
         });
-    if ((threadIdx.x & 63) == 0) {
-      b.dens[i] = make_float2(d0, d1);
-      b.pres[i] = make_float2(p.k * (d0 - p.rho0), p.kn * d1); // sph.h:478-481
-      shCand[w] = cand;
-    }
+      });
+  if ((threadIdx.x & (G - 1)) == 0 && at < n) {
+    b.dens[i] = make_float2(d0, d1);
+    b.pres[i] = make_float2(p.k * (d0 - p.rho0), p.kn * d1);  // sph.h:478-481
   }
-  __syncthreads();
+  uint32_t mn = cand, mx = cand;  // groups past n repeat the last particle
+  block_min_max(mn, mx);
   if (threadIdx.x == 0) {
-    uint32_t mn = 0xFFFFFFFFu, mx = 0u;
-    for (int k = 0; k < kWidePerBlock && (int)(blockIdx.x * kWidePerBlock) + k < n; ++k) {
-      mn = min(mn, shCand[k]);
-      mx = max(mx, shCand[k]);
-    }
     b.candStats[2 * blockIdx.x] = mn;
     b.candStats[2 * blockIdx.x + 1] = mx;
   }
 }
 
-template <bool MULTI>
+template <bool MULTI, int G>
 __global__ __launch_bounds__(kBlock) void k_delta_wide(Buffers b, DevParams p, DevScene s0, int n) {
-  const int i = (int)(blockIdx.x * kWidePerBlock + (threadIdx.x >> 6));
-  if (i >= n) return;  // whole wave
+  __shared__ float4 list[kBlock * kGroupList];
+  const int group = (int)threadIdx.x / G;
+  const int at = (int)(blockIdx.x * kWidePer<G>) + group, i = min(at, n - 1);
   const uint32_t key = b.keys[i];
   const DevScene sc = scene_of_slot<MULTI>(b, s0, key);
   const uint32_t local = key - sc.cellBase;
@@ -1261,33 +1273,41 @@ __global__ __launch_bounds__(kBlock) void k_delta_wide(Buffers b, DevParams p, D
   const int cx = (int)local - cy * sc.nx;
   const float2 xi = b.x1[i];
   const float2 pi = b.pres[i];
-  __shared__ float lds[kWidePerBlock][65 * 4];
+  const float2 pv = b.prev[i];  // requested with the others: at the end it would be one more trip to memory
   float accx = 0.0f, accy = 0.0f;
-  // per pair: accx -= t0, accy -= t1 (demo4.cpp:251), then accx -= t2, accy -= t3
-  // (demo4.cpp:250, j's visit)
-  for_each_pair_wide<4, 2, true>(
-      b.startNext, sc, cx, cy, b.x1, SlotIndex(), xi, p.h2, b.pres, lds[threadIdx.x >> 6], accx, accy,
-      [&](uint32_t, float Rx, float Ry, float r2, float2 pj, float *t) {
+  const bool near = wave_near(p, xi);
+  for_each_pair_wide<G, true>(
+      b.startNext, sc, cx, cy, b.x1, b.pres, (uint32_t)i, xi, p.h2, list + group * (kGroupList * G),
+      [&](float Rx, float Ry, float, float2 pj, float4 &e) {
+        e = make_float4(Rx, Ry, pj.x, pj.y);
+        return true;
+      },
+      [&](float4 e, bool in, int left) {
+        const float r2 = e.x * e.x + e.y * e.y;
         float r, inv;
-        pair_length(r2, r, inv);                                // sph.h:489-490
-        const float nX = Rx * inv, nY = Ry * inv;
+        length_of(near, r2, r, inv);                            // sph.h:489-490
+        const float nX = e.x * inv, nY = e.y * inv;
         const float term = 1.0f - r * p.invH;                   // sph.h:491
         const float tt = term * term;
-        const float dij = p.dt2 * (pi.x * term + pi.y * tt);    // sph.h:492 with P_i
-        const float dji = p.dt2 * (pj.x * term + pj.y * tt);    // sph.h:492 with P_j
-        t[0] = (dij * nX) * 0.5f;
-        t[1] = (dij * nY) * 0.5f;
-        t[2] = (dji * nX) * 0.5f;
-        t[3] = (dji * nY) * 0.5f;
-        return true;
+        const float dij = in ? p.dt2 * (pi.x * term + pi.y * tt) : 0.0f;  // sph.h:492 with P_i
+        const float dji = in ? p.dt2 * (e.z * term + e.w * tt) : 0.0f;    // sph.h:492 with P_j
+        const float t0 = (dij * nX) * 0.5f, t1 = (dij * nY) * 0.5f;
+        const float t2 = (dji * nX) * 0.5f, t3 = (dji * nY) * 0.5f;
+        group_apply<G>(left, [&](auto t) {
+          accx = accx - group_lane<G, decltype(t)::value>(t0);  // demo4.cpp:251
+          accy = accy - group_lane<G, decltype(t)::value>(t1);
+          accx = accx - group_lane<G, decltype(t)::value>(t2);  // demo4.cpp:250 (j's visit)
+          accy = accy - group_lane<G, decltype(t)::value>(t3);
+        });
       });
-  // Every lane holds the same sums: the wave walks the bodies once for lane 0.
+  // Every lane of a group holds the same sums: the wave walks the bodies once
+  // for the groups' first lanes.
+  const bool live = (threadIdx.x & (G - 1)) == 0 && at < n;
   float x = accx + xi.x;                                        // demo4.cpp:253
   float y = accy + xi.y;
-  collide_wave<MULTI>(b, p, sc, x, y, (threadIdx.x & 63) == 0);  // demo4.cpp:411-444
-  if ((threadIdx.x & 63) == 0) {
+  collide_wave<MULTI>(b, p, sc, x, y, live);                    // demo4.cpp:411-444
+  if (live) {
     if (b.dxOut) b.dxOut[i] = make_float2(accx, accy);
-    const float2 pv = b.prev[i];
     b.x0[i] = make_float2(x, y);
     b.v[i] = make_float2((x - pv.x) * p.invDt, (y - pv.y) * p.invDt);  // demo4.cpp:449
   }
@@ -1489,7 +1509,15 @@ __global__ __launch_bounds__(kBlock) void k_selftest_math(const float *a, const 
   out[6 * i + 3] = (float)cell_coord(x, y, 1.0f, 1 << 20);
   float r, inv;
   pair_length(x, r, inv);
-  out[6 * i + 4] = pair_sqrt(x);
+  // both forms of the pair kernels: near_length's where it is used, if it differs
+  float s = pair_sqrt(x);
+  if (x >= 0x1p-96f && x < 0x1p80f) {
+    float ln, li;
+    near_length(x, ln, li);
+    if (ln != s) s = ln;
+    if (li != inv) inv = li;
+  }
+  out[6 * i + 4] = s;
   out[6 * i + 5] = inv;
 }
 
@@ -1518,24 +1546,26 @@ static void visc_cap(const Buffers &b, const DevParams &p, const DevScene &s0, i
                        lists);
 }
 
-static unsigned wide_grid(int n) { return (unsigned)((n + kWidePerBlock - 1) / kWidePerBlock); }
+// Lanes per particle of the wide kernels.
+static int wide_lanes(int n) { return n <= kWideRowParticles ? 16 : 4; }
+static unsigned wide_grid(int n) { return grid_for((uint64_t)n * (uint64_t)wide_lanes(n)); }
 
 uint32_t density_stat_slots(int n, int cap) { return cap == kWideCap ? wide_grid(n) : grid_for(n); }
 
-bool count_in_grid(int n, uint32_t cells, int viscCap) {
-  return viscCap == kWideCap && cells <= kSmallGridCells && n <= kSmallCountParticles;
+uint32_t density_stat_capacity(int n) {
+  return std::max(wide_grid(n), wide_grid(std::min(n, kWideRowParticles)));
 }
 
+bool count_in_grid(int n, uint32_t cells) { return cells <= kSmallGridCells && n <= kSmallCountParticles; }
+
 void launch_visc_predict(const Buffers &b, const DevParams &p, const DevScene &s0, int n, int nBinned, int lists,
-                         int cap, uint32_t cells, hipStream_t s) {
+                         int cap, hipStream_t s) {
   if (n <= 0) return;
   if (cap == kWideCap) {
-    if (b.nScenes > 1)
-      hipLaunchKernelGGL(k_visc_predict_wide<true>, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n, nBinned, lists);
-    else
-      hipLaunchKernelGGL(k_visc_predict_wide<false>, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n, nBinned,
-                         lists);
-    if (!count_in_grid(n, cells, cap)) hipLaunchKernelGGL(k_count_fill, dim3(grid_for(n)), dim3(kBlock), 0, s, b, n);
+    const bool row = wide_lanes(n) == 16, multi = b.nScenes > 1;
+    const auto kern = row ? (multi ? k_visc_predict_wide<true, 16> : k_visc_predict_wide<false, 16>)
+                          : (multi ? k_visc_predict_wide<true, 4> : k_visc_predict_wide<false, 4>);
+    hipLaunchKernelGGL(kern, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n, nBinned, lists);
     return;
   }
   switch (cap) {
@@ -1558,12 +1588,11 @@ void launch_scatter_reorder(const Buffers &b, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_rank_reorder<false>, dim3(grid_for(n)), dim3(kBlock), 0, s, b, n);
 }
 
-bool place_binning(uint32_t cells, int viscCap, bool allBinned) {
-  return cells > kSmallGridCells && viscCap != kWideCap && allBinned;
+bool place_binning(uint64_t n, uint32_t cells, bool allBinned) {
+  return n >= kPlaceMinParticles && cells > kSmallGridCells && allBinned;
 }
 
-uint32_t launch_grid(const Buffers &b, const DevScene &s0, uint32_t cells, int n, int viscCap, bool place,
-                     hipStream_t s) {
+uint32_t launch_grid(const Buffers &b, const DevScene &s0, uint32_t cells, int n, bool place, hipStream_t s) {
   uint32_t slots = 1u;
   if (place) {
     launch_scan(b, cells, n, s);
@@ -1576,12 +1605,14 @@ uint32_t launch_grid(const Buffers &b, const DevScene &s0, uint32_t cells, int n
     }
     return (cells + kScanChunk - 1) / kScanChunk;
   }
-  if (count_in_grid(n, cells, viscCap)) {
+  if (count_in_grid(n, cells)) {
     // counted, scanned and bucketed by one workgroup; the rank pass reads its records
     hipLaunchKernelGGL(k_count_scan_small, dim3(1), dim3(kSmallGridBlock), 0, s, b, n, cells);
     if (n > 0) hipLaunchKernelGGL(k_rank_reorder<true>, dim3(grid_for(n)), dim3(kBlock), 0, s, b, n);
     return slots;
-  } else if (cells <= kSmallGridCells) {
+  }
+  if (n > 0) hipLaunchKernelGGL(k_count_fill, dim3(grid_for(n)), dim3(kBlock), 0, s, b, n);
+  if (cells <= kSmallGridCells) {
     hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kSmallGridBlock), 0, s, b, cells);
   } else {
     Buffers bs = b;
@@ -1604,10 +1635,9 @@ static void density_cap(const Buffers &b, const DevParams &p, const DevScene &s0
 void launch_density(const Buffers &b, const DevParams &p, const DevScene &s0, int n, int cap, hipStream_t s) {
   if (n <= 0) return;
   if (cap == kWideCap) {
-    if (b.nScenes > 1)
-      hipLaunchKernelGGL(k_density_wide<true>, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n);
-    else
-      hipLaunchKernelGGL(k_density_wide<false>, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n);
+    const bool row = wide_lanes(n) == 16, multi = b.nScenes > 1;
+    const auto kern = row ? (multi ? k_density_wide<true, 16> : k_density_wide<false, 16>) : (multi ? k_density_wide<true, 4> : k_density_wide<false, 4>);
+    hipLaunchKernelGGL(kern, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n);
     return;
   }
   switch (cap) {
@@ -1629,10 +1659,9 @@ static void delta_cap(const Buffers &b, const DevParams &p, const DevScene &s0, 
 void launch_delta(const Buffers &b, const DevParams &p, const DevScene &s0, int n, int cap, hipStream_t s) {
   if (n <= 0) return;
   if (cap == kWideCap) {
-    if (b.nScenes > 1)
-      hipLaunchKernelGGL(k_delta_wide<true>, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n);
-    else
-      hipLaunchKernelGGL(k_delta_wide<false>, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n);
+    const bool row = wide_lanes(n) == 16, multi = b.nScenes > 1;
+    const auto kern = row ? (multi ? k_delta_wide<true, 16> : k_delta_wide<false, 16>) : (multi ? k_delta_wide<true, 4> : k_delta_wide<false, 4>);
+    hipLaunchKernelGGL(kern, dim3(wide_grid(n)), dim3(kBlock), 0, s, b, p, s0, n);
     return;
   }
   switch (cap) {

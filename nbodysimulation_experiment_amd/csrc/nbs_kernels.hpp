@@ -114,38 +114,50 @@ void launch_unbin(const Buffers &b, int nBinned, hipStream_t stream);
 // cap: particle positions staged in LDS per workgroup (0, 1024, 2048 or 4096;
 // 0 reads neighbours from global memory).  Every choice gives bit-identical
 // results.
-// cells: the grid's cell count (the counting may move into the grid phase,
-// count_in_grid).
 void launch_visc_predict(const Buffers &b, const DevParams &p, const DevScene &s0, int n, int nBinned, int lists,
-                         int cap, uint32_t cells, hipStream_t stream);
-// Whether the cell counting of a step runs in the grid phase's one-workgroup
-// scan (LDS histogram), which then also buckets the particles, instead of
-// after the viscosity kernel: wide viscosity (viscCap == kWideCap), at most
-// kSmallGridCells cells and kSmallCountParticles particles.
-bool count_in_grid(int n, uint32_t cells, int viscCap);
+                         int cap, hipStream_t stream);
+// Whether one workgroup counts (LDS histogram), scans and buckets the step: at
+// most kSmallGridCells cells and kSmallCountParticles particles.
+bool count_in_grid(int n, uint32_t cells);
 // n: particles (with b.chunkCells set, the scan also fills the chunk table).
 void launch_scan(const Buffers &b, uint32_t cells, int n, hipStream_t stream);
 void launch_scatter_reorder(const Buffers &b, int n, hipStream_t stream);
-// The grid phase: the cell scan (one workgroup for small grids, else
-// launch_scan), then launch_scatter_reorder; with count_in_grid the one
+// The grid phase: k_count_fill and the cell scan (one workgroup for small
+// grids, else launch_scan), then launch_scatter_reorder; with count_in_grid one
 // workgroup counts, scans and buckets, and only the rank pass follows (from
-// its records, b.binRec); with place = true the cell scan and k_place
-// (b.farList etc. set, see place_binning).  Returns the number of
-// (min, max) occupied-cell pairs it leaves in cellStats.
-uint32_t launch_grid(const Buffers &b, const DevScene &s0, uint32_t cells, int n, int viscCap, bool place,
-                     hipStream_t stream);
-// Whether a step can bin by placement (k_place): a grid too large for the
-// one-workgroup scan, the one-lane-per-particle viscosity kernel (which flags
-// the far movers), and every particle binned by the last step.
-bool place_binning(uint32_t cells, int viscCap, bool allBinned);
+// its records, b.binRec); with place = true (the viscosity kernel counted) the
+// cell scan and k_place (b.farList etc. set, see place_binning).  Returns the
+// number of (min, max) occupied-cell pairs it leaves in cellStats.
+uint32_t launch_grid(const Buffers &b, const DevScene &s0, uint32_t cells, int n, bool place, hipStream_t stream);
+// Whether a step bins by placement (k_place): a grid too large for the
+// one-workgroup scan, every particle binned by the last step, and enough
+// particles for its 1,024-slot workgroups to fill the chip.  Two launches and
+// the counts' reread against k_place's ranking by one workgroup per 1,024
+// slots, whole step: 1,048,576 particles 122.4 us placed and 127.0 not;
+// 262,144: 59.3 and 55.1 (collapsed 826 and 795); 65,536: 41.6 and 42.4
+// (collapsed 703 and 671).
+constexpr uint64_t kPlaceMinParticles = 393216;
+bool place_binning(uint64_t n, uint32_t cells, bool allBinned);
 void launch_density(const Buffers &b, const DevParams &p, const DevScene &s0, int n, int cap, hipStream_t stream);
 // Workgroups of the density launch for n particles at capacity cap: the number
 // of (min, max) candidate-count pairs it leaves in candStats.
 uint32_t density_stat_slots(int n, int cap);
+// The most pairs that any density launch of at most n particles leaves.
+uint32_t density_stat_capacity(int n);
 void launch_delta(const Buffers &b, const DevParams &p, const DevScene &s0, int n, int cap, hipStream_t stream);
-// cap value selecting the wide kernels (one wave per particle) of the three
-// pair launchers; results are bit-identical to the other capacities.
+// cap value selecting the wide kernels (several lanes per particle) of the
+// three pair launchers; results are bit-identical to the other capacities.
 constexpr int kWideCap = -1;
+// Lanes per particle of the wide kernels: 16 for at most this many particles
+// (16 lanes each fill the 1,024 SIMDs with one to eight waves), else 4.  Step
+// at 32,400 particles with 16 and with 4: 39.1 and 34.9 us at the 0.5h lattice,
+// 225 and 292 collapsed; at 65,536: 55.9 and 38.8, 519 and 491.
+constexpr int kWideRowParticles = 32768;
+// With the autotuner on, steps of at most this many particles use the wide
+// kernels without timing the others: 65,536 particles 38.8 us against 41.6
+// (tiles of 1,024 or 2,048) at the lattice and 491 against 648 collapsed;
+// 131,044: 57.5 against 46.5, 641 against 701.
+constexpr uint64_t kWideParticles = 65536;
 // The variants the autotuner orders and times (the wide kernels last).
 constexpr int kNumTileCaps = 5;
 constexpr int kTileCaps[kNumTileCaps] = {0, 1024, 2048, 4096, kWideCap};

@@ -393,7 +393,7 @@ class Simulation {
         // Replay pairs of steps (the cell tables and the slot-id arrays
         // alternate between two buffers every step).
         uint32_t pairs = (nsteps - s) / 2;
-        if (tuning_.autotune && tuning_.retune_interval > 0 && n_ >= kTuneMinParticles) {
+        if (tuning_.autotune && tuning_.retune_interval > 0 && !wideStep()) {
           // stop replaying when the next re-tuning is due
           const uint64_t until = tuning_.retune_interval > stepsSinceTune_ ? tuning_.retune_interval - stepsSinceTune_ : 0;
           pairs = std::min<uint32_t>(pairs, (uint32_t)std::max<uint64_t>(1, until / 2));
@@ -722,7 +722,7 @@ class Simulation {
     d_.xp.alloc(cap); d_.x1.alloc(cap); d_.id2.alloc(cap); d_.keyp.alloc(cap); d_.fill.alloc(cap);
     d_.tmpSlot.alloc(cap); d_.binRec.alloc(cap); d_.farList.alloc(cap);
     d_.chunkCells.alloc(2 * ((cap + kPlaceChunk - 1) / kPlaceChunk));
-    d_.candStats.alloc(2 * (size_t)density_stat_slots((int)cap, kWideCap));
+    d_.candStats.alloc(2 * (size_t)density_stat_capacity((int)cap));
     cap_ = cap;
     rebindBuffers();
     destroyGraph();
@@ -869,11 +869,10 @@ class Simulation {
 
   // Pair-kernel variant per phase (viscosity, density, relaxation): an LDS
   // tile capacity, or kWideCap for small steps.
-  // Wide kernels for every phase: below the autotuner's range (a few hundred
-  // particles, where one lane per particle fills a single workgroup) or up to
-  // nbs_tuning.wide_max_particles.
+  // Wide kernels for every phase: below the autotuner's range, where they are
+  // the fastest for every packing, or up to nbs_tuning.wide_max_particles.
   bool wideStep() const {
-    return (tuning_.autotune && n_ < kTuneMinParticles) ||
+    return (tuning_.autotune && n_ <= kWideParticles) ||
            (tuning_.wide_max_particles > 0 && n_ <= (uint64_t)tuning_.wide_max_particles);
   }
   void pairCaps(int cap[3]) const {
@@ -894,7 +893,7 @@ class Simulation {
     // Placement binning: the viscosity kernel lists the far movers, k_place
     // orders and moves; on large grids every step's scan clears the counter
     // of the next step's parity.
-    const bool place = place_binning(totalCells_, cap[0], lists_ && nBinned_ == n_);
+    const bool place = place_binning(n_, totalCells_, lists_ && nBinned_ == n_);
     Buffers bg = buf_;
     bg.farList = place ? d_.farList.p : nullptr;
     bg.chunkCells = place ? d_.chunkCells.p : nullptr;
@@ -906,9 +905,9 @@ class Simulation {
       bg.densTo = sur_->carry.p;
     }
     if (ev >= 0) NBS_HIP(hipEventRecord(events_[5 * ev + 0], stream_));
-    launch_visc_predict(bg, p, s0, n, (int)nBinned_, lists_ ? 1 : 0, cap[0], totalCells_, stream_);
+    launch_visc_predict(bg, p, s0, n, (int)nBinned_, lists_ ? 1 : 0, cap[0], stream_);
     if (ev >= 0) NBS_HIP(hipEventRecord(events_[5 * ev + 1], stream_));
-    cellSlots_ = launch_grid(bg, s0, totalCells_, n, cap[0], place, stream_);
+    cellSlots_ = launch_grid(bg, s0, totalCells_, n, place, stream_);
     if (ev >= 0) NBS_HIP(hipEventRecord(events_[5 * ev + 2], stream_));
     if (!carried) {
       launch_density(buf_, p, s0, n, cap[1], stream_);
@@ -930,14 +929,13 @@ class Simulation {
   // Each of kTuneReps rounds runs one step per candidate; each kernel keeps
   // its fastest candidate (minimum over rounds).
   static constexpr uint32_t kTuneReps = 2;
-  static constexpr uint64_t kTuneMinParticles = 1024;
-  // The wide kernels (one wave per particle) are a candidate only for steps
-  // small enough that one lane per particle leaves the chip idle.
+  // The wide kernels (four lanes per particle here) are a candidate only for
+  // steps small enough that one lane per particle leaves the chip idle.
   static constexpr uint64_t kWideTuneMax = 131072;
   int numCaps() const { return n_ <= kWideTuneMax ? kNumTileCaps : kNumTileCaps - 1; }
   uint32_t tuneVariants() const { return tuned_ ? 3u : (uint32_t)numCaps(); }
   bool wantTune() const {
-    if (!tuning_.autotune || n_ < kTuneMinParticles || !lists_ || nBinned_ != n_ || surrogateMode() || wideStep())
+    if (!tuning_.autotune || !lists_ || nBinned_ != n_ || surrogateMode() || wideStep())
       return false;
     return !tuned_ || (tuning_.retune_interval > 0 && stepsSinceTune_ >= tuning_.retune_interval);
   }
@@ -1176,7 +1174,7 @@ class Simulation {
     S.densA.alloc(c);
     S.densB.alloc(c);
     S.presScratch.alloc(c);
-    S.candScratch.alloc(2 * (size_t)density_stat_slots((int)c, kWideCap));
+    S.candScratch.alloc(2 * (size_t)density_stat_capacity((int)c));
     S.errPartials.alloc(2 * std::max<size_t>((c + 2047) / 2048, 1));
     S.errOut.alloc(2);
     S.pairPart.alloc(surrogate_forward_waves((int)c));

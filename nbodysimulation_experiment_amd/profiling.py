@@ -44,9 +44,9 @@ SHORT = [
 # group lists its alternatives: the kernels one step launches for the phase in
 # the one-lane-per-particle and in the wide form.
 GROUPS = {
-    "viscosity_predict": (("viscosity_predict",), ("viscosity_predict_wide", "count_fill"), ("viscosity_predict_wide",)),
-    "grid": (("scan_reduce", "scan_final", "place"), ("scan_reduce", "scan_final", "scatter", "rank_reorder"),
-             ("scan_small", "scatter", "rank_reorder"), ("count_scan_small", "scatter", "rank_reorder")),
+    "viscosity_predict": (("viscosity_predict",), ("viscosity_predict_wide",)),
+    "grid": (("scan_reduce", "scan_final", "place"), ("count_fill", "scan_reduce", "scan_final", "scatter", "rank_reorder"),
+             ("count_fill", "scan_small", "scatter", "rank_reorder"), ("count_scan_small", "rank_reorder")),
     "density": (("density",), ("density_wide",)),
     "delta": (("delta",), ("delta_wide",)),
     "surrogate_forward": (("sur_forward",),),
