@@ -1335,6 +1335,28 @@ __global__ __launch_bounds__(kBlock) void k_gather_state(Buffers b, DevScene s0,
   }
 }
 
+// Restores positions and velocities in particle-index order (slots = indices):
+// prev = x, no own acceleration, density or pressure, the cell of the restored
+// position; scene is read when there are several.
+__global__ __launch_bounds__(kBlock) void k_set_state(Buffers b, DevScene s0, int n, const float2 *x, const float2 *v,
+                                                      const int32_t *scene) {
+  const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
+  if (i >= n) return;
+  const int s = b.nScenes > 1 ? scene[i] : 0;
+  const DevScene sc = b.nScenes > 1 ? b.scenes[s] : s0;
+  const float2 p = x[i], zero = make_float2(0.0f, 0.0f);
+  const int cx = cell_coord(p.x, sc.halfW, sc.cellSize, sc.nx), cy = cell_coord(p.y, sc.halfH, sc.cellSize, sc.ny);
+  b.x0[i] = p;
+  b.prev[i] = p;
+  b.v[i] = v[i];
+  b.acc[i] = zero;
+  b.dens[i] = zero;
+  b.pres[i] = zero;
+  b.id[i] = (uint32_t)i;
+  b.keys[i] = sc.cellBase + (uint32_t)(cy * sc.nx + cx);
+  b.scn[i] = (uint32_t)s;
+}
+
 // sph.h:683-695 SPHGetParticleColor, in particle-index order.  The clamps
 // keep std::min / std::max's comparison order (NaN passes through).
 __global__ __launch_bounds__(kBlock) void k_colors(Buffers b, float rho0, int n, float4 *rgba) {
@@ -1677,6 +1699,12 @@ void launch_gather_state(const Buffers &b, const DevScene &s0, int n, int nBinne
   if (n <= 0) return;
   hipLaunchKernelGGL(k_gather_state, dim3(grid_for(n)), dim3(kBlock), 0, s, b, s0, n, nBinned, x, prev, v, dens, pres,
                      key, scene);
+}
+
+void launch_set_state(const Buffers &b, const DevScene &s0, int n, const float2 *x, const float2 *v,
+                      const int32_t *scene, hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_set_state, dim3(grid_for(n)), dim3(kBlock), 0, s, b, s0, n, x, v, scene);
 }
 
 void launch_colors(const Buffers &b, float rho0, int n, float4 *rgba, hipStream_t s) {

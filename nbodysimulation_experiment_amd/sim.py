@@ -35,6 +35,38 @@ def _f32(a, cols=2):
     return a.reshape(-1, cols) if cols else a
 
 
+# Arrays that the library fills completely, adjacent in blocks of at most this
+# many bytes: one device copy per block, and the C library's allocator hands a
+# freed block out again (below its 32 MiB limit for separately mapped blocks)
+# instead of mapping fresh pages, whose first writes cost more than the copy
+# (its heap keeps up to twice the largest block freed so far, so a state's
+# first block is made the larger one: 28 of 48 bytes a particle).
+_HOST_BLOCK = 28 << 20
+
+
+def _host_arrays(fields: dict) -> dict:
+    """{name: (rows, cols or 0, dtype)} -> uninitialised arrays."""
+    out, group, size = {}, [], 0
+
+    def carve():
+        block, at = np.empty(size, np.uint8), 0
+        for name, (rows, cols, dtype), nbytes in group:
+            a = block[at:at + nbytes].view(dtype)
+            out[name] = a.reshape(rows, cols) if cols else a
+            at += nbytes
+
+    for name, f in fields.items():
+        nbytes = f[0] * max(f[1], 1) * np.dtype(f[2]).itemsize
+        if group and size + nbytes > _HOST_BLOCK:
+            carve()
+            group, size = [], 0
+        group.append((name, f, nbytes))
+        size += nbytes
+    if group:
+        carve()
+    return out
+
+
 def params_to_c(p: SPHParams, cell_size: float = 1.0, particle_spacing: float | None = None) -> NbsParams:
     spacing = p.h * 0.5 if particle_spacing is None else particle_spacing
     return NbsParams(p.h, cell_size, spacing, p.rho0, p.k, p.k_near, p.sigma, p.beta, p.collision_radius,
@@ -231,16 +263,17 @@ class ParticleSimulation:
 
     def get_state(self) -> dict:
         n = self.GetParticleCount()
-        out = {k: np.zeros((n, 2), np.float32) for k in ("x", "prev", "v", "density", "pressure")}
-        out["key"] = np.zeros(n, np.uint32)
-        out["scene"] = np.zeros(n, np.int32)
+        out = _host_arrays({"x": (n, 2, np.float32), "prev": (n, 2, np.float32), "v": (n, 2, np.float32),
+                            "key": (n, 0, np.uint32), "density": (n, 2, np.float32), "pressure": (n, 2, np.float32),
+                            "scene": (n, 0, np.int32)})
+        out = {k: out[k] for k in ("x", "prev", "v", "density", "pressure", "key", "scene")}
         call("nbs_get_state", self._h, _ptr(out["x"]), _ptr(out["prev"]), _ptr(out["v"]), _ptr(out["density"]),
              _ptr(out["pressure"]), _ptr(out["key"]), _ptr(out["scene"]))
         return out
 
     def get_colors(self) -> np.ndarray:
         """Per-particle RGBA of the reference's Render (sph.h:683-695), particle-index order."""
-        out = np.zeros((self.GetParticleCount(), 4), np.float32)
+        out = np.empty((self.GetParticleCount(), 4), np.float32)
         call("nbs_get_colors", self._h, _ptr(out))
         return out
 
@@ -356,15 +389,16 @@ class ParticleSimulation:
         cap = n0 + 4096  # room for particles an emitter adds during the step
         grad = np.zeros(_lib.SURROGATE_WEIGHT_COUNT, np.float32)
         loss = np.zeros(1, np.float32)
-        arrs = {k: np.zeros((cap, 2), np.float32) for k in ("out", "x", "prev", "density", "target")}
-        scene = np.zeros(cap, np.int32)
+        arrs = _host_arrays({**{k: (cap, 2, np.float32) for k in ("out", "x", "prev", "density", "target")},
+                             "scene": (cap, 0, np.int32)})
+        scene = arrs.pop("scene")
         call("nbs_surrogate_frame", self._h, float(dt), _ptr(grad), _ptr(loss), _ptr(arrs["out"]), _ptr(arrs["x"]),
              _ptr(arrs["prev"]), _ptr(arrs["density"]), _ptr(arrs["target"]), _ptr(scene))
         n = self.GetParticleCount()
         if n > cap:
             raise RuntimeError("an emitter added more particles than the frame buffers hold")
-        res = {k: v[:n].copy() for k, v in arrs.items()}
-        res.update(grad=grad, loss=float(loss[0]), scene=scene[:n].copy())
+        res = {k: v[:n] for k, v in arrs.items()}
+        res.update(grad=grad, loss=float(loss[0]), scene=scene[:n])
         return res
 
 
