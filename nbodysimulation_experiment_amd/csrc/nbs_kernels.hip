@@ -30,6 +30,27 @@
 
 namespace nbs {
 
+// Whether near_length serves this wave's active lanes: h > 2^-36, and no
+// particle with |x| or |y| below 2^-23 (two different floats of which one is
+// 2^-23 or more differ by 2^-47 or more, so every pair of such a particle has
+// r2 == 0 or r2 >= 2^-96).
+__device__ __forceinline__ bool wave_near(const DevParams &p, float2 x) {
+  return p.h > 0x1p-36f && __ballot(fminf(fabsf(x.x), fabsf(x.y)) < 0x1p-23f) == 0ull;
+}
+// The pair length by near_length or pair_length; near is wave-uniform, and a
+// compile-time constant in the one-lane-per-particle walks, whose four slots
+// then share one block without branches.  pair_length's branch for tiny r2 was
+// taken by nearly every wave there, since r2 == 0 for a particle and itself:
+// 1,048,576 particles (step 480) viscosity 91 -> 76 us, density 61 -> 54, delta
+// 91 -> 77.
+__device__ __forceinline__ void length_of(bool near, float r2, float &r, float &inv) {
+  if (near)
+    near_length(r2, r, inv);
+  else
+    pair_length(r2, r, inv);
+}
+__device__ __forceinline__ float root_of(bool near, float r2) { return near ? near_sqrt(r2) : pair_sqrt(r2); }
+
 // For every candidate slot j of the particle at xi in cell (cx, cy) whose
 // r2 < h2 (sph.h:470, 488, 502), in candidate order, applies the pair's
 // contribution: apply(term(j, Rx, Ry, r2, true)).  term(..., false) must return
@@ -253,20 +274,6 @@ __device__ __forceinline__ uint32_t wave_aggregated_fill(uint32_t *count, uint32
   return base + rank;
 }
 
-// Whether near_length serves this wave's active lanes: h > 2^-36, and no
-// particle with |x| or |y| below 2^-23 (two different floats of which one is
-// 2^-23 or more differ by 2^-47 or more, so every pair of such a particle has
-// r2 == 0 or r2 >= 2^-96).
-__device__ __forceinline__ bool wave_near(const DevParams &p, float2 x) {
-  return p.h > 0x1p-36f && __ballot(fminf(fabsf(x.x), fabsf(x.y)) < 0x1p-23f) == 0ull;
-}
-__device__ __forceinline__ void length_of(bool near, float r2, float &r, float &inv) {
-  if (near)  // wave-uniform
-    near_length(r2, r, inv);
-  else
-    pair_length(r2, r, inv);
-}
-
 // Appends `value` of every lane with `flag` to list[*counter ...] with one
 // atomic per wave; entries at cap or beyond are dropped.  All active lanes must
 // call it.
@@ -304,26 +311,28 @@ __device__ __forceinline__ void put_key(const Buffers &b, uint32_t key, bool far
 // ---------------------------------------------------------------------------
 // demo4.cpp:223-237 in Jacobi order: both halves of each pair's impulse from
 // the integrated velocities (neighbours have no own acceleration: v_j + g dt).
-template <typename Idx>
+template <bool NEAR, typename Idx>
 __device__ __forceinline__ void viscosity_sum(const uint32_t *start, const DevScene &sc, int cx, int cy,
                                               const float2 *X, const float2 *V, Idx idx, const DevParams &p,
                                               float2 xi, float vx, float vy, float &accx, float &accy) {
+  const float invH = in_vgpr(p.invH), sigma = in_vgpr(p.sigma), beta = in_vgpr(p.beta), dt = in_vgpr(p.dt);
+  const float gx = in_vgpr(p.gdtx), gy = in_vgpr(p.gdty);
   for_each_pair(
       start, sc, cx, cy, X, idx, xi, p.h2,
       [&](uint32_t j, float Rx, float Ry, float r2, bool use) {
         const float2 vj = V[j];
-        const float vjx = p.gdtx + vj.x, vjy = p.gdty + vj.y;
+        const float vjx = gx + vj.x, vjy = gy + vj.y;
         float r, inv;
-        pair_length(r2, r, inv);                          // sph.h:503, 505 Vec2Normalize (length 0 -> 1)
-        const float qq = r * p.invH;                      // sph.h:504
+        length_of(NEAR, r2, r, inv);                      // sph.h:503, 505 Vec2Normalize (length 0 -> 1)
+        const float qq = r * invH;                        // sph.h:504
         const float nX = Rx * inv, nY = Ry * inv;
         const float u = (vx - vjx) * nX + (vy - vjy) * nY;  // sph.h:506
         // no impulse unless u > 0 (sph.h:507): a zero force times the finite
         // normal, 0.5 and dt gives +0 or -0, and subtracting either leaves the
         // sums unchanged (they start at +0 and never hold -0)
-        const float f = (use && u > 0.0f) ? (1.0f - qq) * (p.sigma * u + p.beta * (u * u)) : 0.0f;  // sph.h:508
-        const float ix = ((f * nX) * 0.5f) * p.dt;       // demo4.cpp:233 force * 0.5f * deltaTime
-        const float iy = ((f * nY) * 0.5f) * p.dt;
+        const float f = (use && u > 0.0f) ? (1.0f - qq) * (sigma * u + beta * (u * u)) : 0.0f;  // sph.h:508
+        const float ix = ((f * nX) * 0.5f) * dt;         // demo4.cpp:233 force * 0.5f * deltaTime
+        const float iy = ((f * nY) * 0.5f) * dt;
         return make_float2(ix, iy);
       },
       [&](float2 im) {
@@ -381,10 +390,13 @@ __global__ __launch_bounds__(kBlock) void k_visc_predict(Buffers b, DevParams p,
     pcy = (int)(local / (uint32_t)sc.nx);
     pcx = (int)local - pcy * sc.nx;
     float accx = 0.0f, accy = 0.0f;
-    if (CAP > 0 && plan.use)
-      viscosity_sum(b.startCur, sc, pcx, pcy, tx, b.v, TileIndex(plan), p, xi, vx, vy, accx, accy);
+    const bool near = wave_near(p, xi);
+    if (CAP > 0 && plan.use && near)
+      viscosity_sum<true>(b.startCur, sc, pcx, pcy, tx, b.v, TileIndex(plan), p, xi, vx, vy, accx, accy);
+    else if (near)
+      viscosity_sum<true>(b.startCur, sc, pcx, pcy, b.x0, b.v, SlotIndex(), p, xi, vx, vy, accx, accy);
     else
-      viscosity_sum(b.startCur, sc, pcx, pcy, b.x0, b.v, SlotIndex(), p, xi, vx, vy, accx, accy);
+      viscosity_sum<false>(b.startCur, sc, pcx, pcy, b.x0, b.v, SlotIndex(), p, xi, vx, vy, accx, accy);
     vx = accx + vx;
     vy = accy + vy;
   }
@@ -986,17 +998,18 @@ __global__ __launch_bounds__(kSmallGridBlock) void k_count_scan_small(Buffers b,
 // ---------------------------------------------------------------------------
 // 4. density + pressure
 // ---------------------------------------------------------------------------
-template <typename Idx>
+template <bool NEAR, typename Idx>
 __device__ __forceinline__ uint32_t density_sum(const uint32_t *start, const DevScene &sc, int cx, int cy,
                                                 const float2 *X, Idx idx, const DevParams &p, float2 xi, float &d0,
                                                 float &d1) {
+  const float invH = in_vgpr(p.invH);
   return for_each_pair(
       start, sc, cx, cy, X, idx, xi, p.h2,
       [&](uint32_t, float, float, float r2, bool use) {
-        const float r = pair_sqrt(r2);                    // sph.h:471
+        const float r = root_of(NEAR, r2);                // sph.h:471
         // term +0 gives terms +0: adding them leaves the sums unchanged (they
         // start at +0 and never hold -0)
-        const float term = use ? 1.0f - r * p.invH : 0.0f;  // sph.h:472
+        const float term = use ? 1.0f - r * invH : 0.0f;  // sph.h:472
         const float t2 = term * term, t3 = (term * term) * term;
         return make_float2(t2, t3);
       },
@@ -1036,10 +1049,13 @@ __global__ __launch_bounds__(kBlock) void k_density(Buffers b, DevParams p, DevS
     const int cx = (int)local - cy * sc.nx;
     const float2 xi = b.x1[i];
     float d0 = 0.0f, d1 = 0.0f;
-    if (CAP > 0 && plan.use)
-      cand = density_sum(b.startNext, sc, cx, cy, tx, TileIndex(plan), p, xi, d0, d1);
+    const bool near = wave_near(p, xi);
+    if (CAP > 0 && plan.use && near)
+      cand = density_sum<true>(b.startNext, sc, cx, cy, tx, TileIndex(plan), p, xi, d0, d1);
+    else if (near)
+      cand = density_sum<true>(b.startNext, sc, cx, cy, b.x1, SlotIndex(), p, xi, d0, d1);
     else
-      cand = density_sum(b.startNext, sc, cx, cy, b.x1, SlotIndex(), p, xi, d0, d1);
+      cand = density_sum<false>(b.startNext, sc, cx, cy, b.x1, SlotIndex(), p, xi, d0, d1);
     b.dens[i] = make_float2(d0, d1);
     b.pres[i] = make_float2(p.k * (d0 - p.rho0), p.kn * d1);  // sph.h:478-481
   }
@@ -1058,24 +1074,25 @@ __global__ __launch_bounds__(kBlock) void k_density(Buffers b, DevParams p, DevS
 // ---------------------------------------------------------------------------
 // demo4.cpp:239-255 in Jacobi order: -delta_ij/2 from the particle's own visit
 // and +delta_ji/2 from the neighbour's visit (n_ji = -n_ij).
-template <typename Idx>
+template <bool NEAR, typename Idx>
 __device__ __forceinline__ void delta_sum(const uint32_t *start, const DevScene &sc, int cx, int cy, const float2 *X,
                                           const float2 *P, Idx idx, const DevParams &p, float2 xi, float2 pi,
                                           float &accx, float &accy) {
+  const float invH = in_vgpr(p.invH), dt2 = in_vgpr(p.dt2);
   for_each_pair(
       start, sc, cx, cy, X, idx, xi, p.h2,
       [&](uint32_t j, float Rx, float Ry, float r2, bool use) {
         const float2 pj = P[j];
         float r, inv;
-        pair_length(r2, r, inv);                          // sph.h:489-490 Vec2Normalize (length 0 -> 1)
+        length_of(NEAR, r2, r, inv);                      // sph.h:489-490 Vec2Normalize (length 0 -> 1)
         const float nX = Rx * inv, nY = Ry * inv;
-        const float term = 1.0f - r * p.invH;             // sph.h:491
+        const float term = 1.0f - r * invH;               // sph.h:491
         const float tt = term * term;
         // a zero displacement times the finite normal and 0.5 gives +0 or -0,
         // and subtracting either leaves the sums unchanged (they start at +0
         // and never hold -0)
-        const float dij = use ? p.dt2 * (pi.x * term + pi.y * tt) : 0.0f;  // sph.h:492 with P_i
-        const float dji = use ? p.dt2 * (pj.x * term + pj.y * tt) : 0.0f;  // sph.h:492 with P_j (j's visit)
+        const float dij = use ? dt2 * (pi.x * term + pi.y * tt) : 0.0f;  // sph.h:492 with P_i
+        const float dji = use ? dt2 * (pj.x * term + pj.y * tt) : 0.0f;  // sph.h:492 with P_j (j's visit)
         return make_float4((dij * nX) * 0.5f, (dij * nY) * 0.5f, (dji * nX) * 0.5f, (dji * nY) * 0.5f);
       },
       [&](float4 d) {
@@ -1111,10 +1128,13 @@ __global__ __launch_bounds__(kBlock) void k_delta(Buffers b, DevParams p, DevSce
     const float2 xi = b.x1[i];
     const float2 pi = b.pres[i];
     float accx = 0.0f, accy = 0.0f;
-    if (CAP > 0 && plan.use)
-      delta_sum(b.startNext, sc, cx, cy, tx, b.pres, TileIndex(plan), p, xi, pi, accx, accy);
+    const bool near = wave_near(p, xi);
+    if (CAP > 0 && plan.use && near)
+      delta_sum<true>(b.startNext, sc, cx, cy, tx, b.pres, TileIndex(plan), p, xi, pi, accx, accy);
+    else if (near)
+      delta_sum<true>(b.startNext, sc, cx, cy, b.x1, b.pres, SlotIndex(), p, xi, pi, accx, accy);
     else
-      delta_sum(b.startNext, sc, cx, cy, b.x1, b.pres, SlotIndex(), p, xi, pi, accx, accy);
+      delta_sum<false>(b.startNext, sc, cx, cy, b.x1, b.pres, SlotIndex(), p, xi, pi, accx, accy);
     if (b.dxOut) b.dxOut[i] = make_float2(accx, accy);
     x = accx + xi.x;                                      // demo4.cpp:253
     y = accy + xi.y;

@@ -52,12 +52,15 @@ def test_crowded_lists_with_both_group_widths(side, box):
     _check(spec, SPHParams(k=0.0005, k_near=0.001), (0.0, -9.8), [1, 4])
 
 
-def test_coordinates_near_zero_and_far_outside():
-    # |x| below 2^-23 takes the square root's form for tiny operands; particles outside the grid share its border cells
-    pos = volume_positions((0.0, 0.0), 20, 20, 0.4, 1.0, seed=5)
+@pytest.mark.parametrize("side,box,h", [(20, 24.0, 1.0), (260, 130.0, 1.0), (260, 130.0, 2.0 ** -37)])
+def test_coordinates_near_zero_and_far_outside(side, box, h):
+    # |x| below 2^-23, and h below 2^-36, take the square root's form for tiny operands (260 x 260: the
+    # one-lane-per-particle kernels, from the staged and the global positions);
+    # particles outside the grid share its border cells
+    pos = volume_positions((0.0, 0.0), side, side, 0.4, 1.0, seed=5)
     pos[:6] = [(0.0, 0.0), (1e-20, -1e-20), (1e-30, 0.2), (1e-7, 1e-9), (400.0, 3.0), (400.2, 3.1)]
-    spec = SceneSpec(24.0, 24.0, 1.0, pos, planes=[])
-    _check(spec, SPHParams(sigma=0.2), (0.0, 0.0), [1, 5])
+    spec = SceneSpec(box, box, 1.0, pos, planes=[])
+    _check(spec, SPHParams(h=h, sigma=0.2), (0.0, 0.0), [1, 5])
 
 
 def test_placement_from_its_smallest_step_on():
