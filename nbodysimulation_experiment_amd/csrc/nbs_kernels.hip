@@ -51,7 +51,43 @@ __device__ __forceinline__ void length_of(bool near, float r2, float &r, float &
 }
 __device__ __forceinline__ float root_of(bool near, float r2) { return near ? near_sqrt(r2) : pair_sqrt(r2); }
 
-// For every candidate slot j of the particle at xi in cell (cx, cy) whose
+// What a workgroup's pair walk starts from: the tile plan of its slots
+// [i0, min(i0 + kBlock, end)), whose first and last cell bound the others', and
+// the calling particle's scene, cell and rows (key: its cell).  Every wave
+// plans for itself in scalar registers, so the plan needs no barrier, and the
+// particle's rows are requested before the tile is staged: keys, cell starts
+// and tile are three memory round trips, where a plan left in LDS by one thread
+// and rows read after the tile took five.  A slot range within one scene reads
+// that scene once.  96 scenes, 1.76 M particles: viscosity 66.6 -> 62.5 us,
+// density 45.2 -> 41.9, delta 61.5 -> 60; one scene of 1,048,576: unchanged
+// (its kernels are bound by the walk's issue: of 38.5 us viscosity, 17 remain
+// without the walk, 25 with the walk's tests alone).
+template <bool MULTI, int CAP>
+__device__ __forceinline__ void open_block(const Buffers &b, const DevScene &s0, const uint32_t *start, int i0,
+                                           int end, uint32_t key, DevScene &sc, TilePlan &plan, int &cx, int &cy,
+                                           RowRange (&rows)[3]) {
+  const uint32_t kA = (uint32_t)__builtin_amdgcn_readfirstlane((int)b.keys[i0]);
+  const uint32_t kB = (uint32_t)__builtin_amdgcn_readfirstlane((int)b.keys[min(i0 + kBlock, end) - 1]);
+  if (MULTI) {
+    const int a = __builtin_amdgcn_readfirstlane(scene_index(b, kA));
+    const int e = __builtin_amdgcn_readfirstlane(scene_index(b, kB));
+    sc = b.scenes[a];
+    plan_tile<CAP>(start, sc, kA, kB, plan);
+    if (a != e) {
+      plan.use = 0;
+      sc = b.scenes[scene_index(b, key)];
+    }
+  } else {
+    sc = s0;
+    plan_tile<CAP>(start, sc, kA, kB, plan);
+  }
+  const uint32_t local = key - sc.cellBase;
+  cy = (int)(local / (uint32_t)sc.nx);
+  cx = (int)local - cy * sc.nx;
+  row_ranges(start, sc, cx, cy, rows);
+}
+
+// For every candidate slot j (of the three row ranges) of the particle at xi whose
 // r2 < h2 (sph.h:470, 488, 502), in candidate order, applies the pair's
 // contribution: apply(term(j, Rx, Ry, r2, true)).  term(..., false) must return
 // a contribution that leaves the accumulators unchanged bit for bit.
@@ -64,12 +100,9 @@ __device__ __forceinline__ float root_of(bool near, float r2) { return near ? ne
 constexpr int kPairsPerIter = 4;
 
 template <typename Idx, typename Term, typename Apply>
-__device__ __forceinline__ uint32_t for_each_pair(const uint32_t *start, const DevScene &sc, int cx, int cy,
-                                                  const float2 *X, Idx idx, float2 xi, float h2, Term &&term,
-                                                  Apply &&apply) {
+__device__ __forceinline__ uint32_t for_each_pair(const RowRange (&rows)[3], const float2 *X, Idx idx, float2 xi,
+                                                  float h2, Term &&term, Apply &&apply) {
   uint32_t cand = 0;
-  RowRange rows[3];
-  row_ranges(start, sc, cx, cy, rows);
   for (int d = 0; d < 3; ++d) {
     const RowRange rr = rows[d];
     cand += rr.j1 - rr.j0;
@@ -312,13 +345,13 @@ __device__ __forceinline__ void put_key(const Buffers &b, uint32_t key, bool far
 // demo4.cpp:223-237 in Jacobi order: both halves of each pair's impulse from
 // the integrated velocities (neighbours have no own acceleration: v_j + g dt).
 template <bool NEAR, typename Idx>
-__device__ __forceinline__ void viscosity_sum(const uint32_t *start, const DevScene &sc, int cx, int cy,
-                                              const float2 *X, const float2 *V, Idx idx, const DevParams &p,
-                                              float2 xi, float vx, float vy, float &accx, float &accy) {
+__device__ __forceinline__ void viscosity_sum(const RowRange (&rows)[3], const float2 *X, const float2 *V, Idx idx,
+                                              const DevParams &p, float2 xi, float vx, float vy, float &accx,
+                                              float &accy) {
   const float invH = in_vgpr(p.invH), sigma = in_vgpr(p.sigma), beta = in_vgpr(p.beta), dt = in_vgpr(p.dt);
   const float gx = in_vgpr(p.gdtx), gy = in_vgpr(p.gdty);
   for_each_pair(
-      start, sc, cx, cy, X, idx, xi, p.h2,
+      rows, X, idx, xi, p.h2,
       [&](uint32_t j, float Rx, float Ry, float r2, bool use) {
         const float2 vj = V[j];
         const float vjx = gx + vj.x, vjy = gy + vj.y;
@@ -347,56 +380,49 @@ template <bool MULTI, int CAP>
 __global__ __launch_bounds__(kBlock) void k_visc_predict(Buffers b, DevParams p, DevScene s0, int n, int nBinned,
                                                          int lists) {
   __shared__ float2 tx[CAP > 0 ? CAP : 1];
-  __shared__ TilePlan plan;
   const int i0 = (int)(blockIdx.x * kBlock);
   const int i = i0 + (int)threadIdx.x;
+  const bool binned = i < nBinned;
+  const int il = min(i, n - 1);
+  const float2 xi = b.x0[il];
+  const float2 vi = b.v[il];
   // Viscosity runs for slots of the previous binning when lists exist.
   const bool tileVisc = lists && i0 < nBinned;
+  TilePlan plan;
+  DevScene sc = s0;
+  int pcx = -2, pcy = -2;  // cell of the last binning (none: not adjacent to any cell)
+  RowRange rows[3];
   if (tileVisc) {
-    if (threadIdx.x == 0) {
-      const uint32_t kA = b.keys[i0], kB = b.keys[min(i0 + kBlock, nBinned) - 1];
-      const DevScene sa = scene_of_slot<MULTI>(b, s0, kA);
-      plan_tile<CAP>(b.startCur, sa, kA, kB, plan);
-      if (MULTI && sa.cellBase != scene_of_slot<MULTI>(b, s0, kB).cellBase) plan.use = 0;
-    }
+    open_block<MULTI, CAP>(b, s0, b.startCur, i0, nBinned, b.keys[min(i, nBinned - 1)], sc, plan, pcx, pcy, rows);
+    if (CAP > 0 && plan.use) stage(plan, b.x0, tx);
     __syncthreads();
-    if (CAP > 0 && plan.use) {
-      stage(plan, b.x0, tx);
-    }
-    __syncthreads();
+  } else if (MULTI && binned) {
+    sc = scene_of_slot<MULTI>(b, s0, b.keys[i]);
   }
   if (i >= n) return;
-  const float2 xi = b.x0[i];
-  const float2 vi = b.v[i];
-  const bool binned = i < nBinned;
   float aX, aY;
-  DevScene sc;
   if (binned) {
     aX = p.gex + 0.0f;                                   // demo4.cpp:306 (own acceleration is zero)
     aY = p.gey + 0.0f;
-    sc = scene_of_slot<MULTI>(b, s0, b.keys[i]);
   } else {
     const float2 a = b.acc[i];
     aX = p.gex + a.x;
     aY = p.gey + a.y;
-    sc = MULTI ? b.scenes[b.scn[i]] : s0;
+    if (MULTI) sc = b.scenes[b.scn[i]];
+    pcx = pcy = -2;
   }
   float vx = (aX * p.dt) + vi.x;                         // demo4.cpp:307
   float vy = (aY * p.dt) + vi.y;
 
-  int pcx = -2, pcy = -2;  // cell of the last binning (none: not adjacent to any cell)
   if (lists && binned) {
-    const uint32_t local = b.keys[i] - sc.cellBase;
-    pcy = (int)(local / (uint32_t)sc.nx);
-    pcx = (int)local - pcy * sc.nx;
     float accx = 0.0f, accy = 0.0f;
     const bool near = wave_near(p, xi);
     if (CAP > 0 && plan.use && near)
-      viscosity_sum<true>(b.startCur, sc, pcx, pcy, tx, b.v, TileIndex(plan), p, xi, vx, vy, accx, accy);
+      viscosity_sum<true>(rows, tx, b.v, TileIndex(plan), p, xi, vx, vy, accx, accy);
     else if (near)
-      viscosity_sum<true>(b.startCur, sc, pcx, pcy, b.x0, b.v, SlotIndex(), p, xi, vx, vy, accx, accy);
+      viscosity_sum<true>(rows, b.x0, b.v, SlotIndex(), p, xi, vx, vy, accx, accy);
     else
-      viscosity_sum<false>(b.startCur, sc, pcx, pcy, b.x0, b.v, SlotIndex(), p, xi, vx, vy, accx, accy);
+      viscosity_sum<false>(rows, b.x0, b.v, SlotIndex(), p, xi, vx, vy, accx, accy);
     vx = accx + vx;
     vy = accy + vy;
   }
@@ -999,12 +1025,11 @@ __global__ __launch_bounds__(kSmallGridBlock) void k_count_scan_small(Buffers b,
 // 4. density + pressure
 // ---------------------------------------------------------------------------
 template <bool NEAR, typename Idx>
-__device__ __forceinline__ uint32_t density_sum(const uint32_t *start, const DevScene &sc, int cx, int cy,
-                                                const float2 *X, Idx idx, const DevParams &p, float2 xi, float &d0,
-                                                float &d1) {
+__device__ __forceinline__ uint32_t density_sum(const RowRange (&rows)[3], const float2 *X, Idx idx,
+                                                const DevParams &p, float2 xi, float &d0, float &d1) {
   const float invH = in_vgpr(p.invH);
   return for_each_pair(
-      start, sc, cx, cy, X, idx, xi, p.h2,
+      rows, X, idx, xi, p.h2,
       [&](uint32_t, float, float, float r2, bool use) {
         const float r = root_of(NEAR, r2);                // sph.h:471
         // term +0 gives terms +0: adding them leaves the sums unchanged (they
@@ -1019,43 +1044,30 @@ __device__ __forceinline__ uint32_t density_sum(const uint32_t *start, const Dev
       });
 }
 
-// Plans the tile of the workgroup at slots [i0, i0 + kBlock) of the new binning.
-template <bool MULTI, int CAP>
-__device__ __forceinline__ void plan_new(const Buffers &b, const DevScene &s0, int i0, int n, TilePlan &plan) {
-  if (threadIdx.x == 0) {
-    const uint32_t kA = b.keys[i0], kB = b.keys[min(i0 + kBlock, n) - 1];
-    const DevScene sa = scene_of_slot<MULTI>(b, s0, kA);
-    plan_tile<CAP>(b.startNext, sa, kA, kB, plan);
-    if (MULTI && sa.cellBase != scene_of_slot<MULTI>(b, s0, kB).cellBase) plan.use = 0;
-  }
-  __syncthreads();
-}
-
 template <bool MULTI, int CAP>
 __global__ __launch_bounds__(kBlock) void k_density(Buffers b, DevParams p, DevScene s0, int n) {
   __shared__ float2 tx[CAP > 0 ? CAP : 1];
-  __shared__ TilePlan plan;
   const int i0 = (int)(blockIdx.x * kBlock);
   const int i = i0 + (int)threadIdx.x;
-  plan_new<MULTI, CAP>(b, s0, i0, n, plan);
+  const int il = min(i, n - 1);
+  const float2 xi = b.x1[il];
+  TilePlan plan;
+  DevScene sc;
+  int cx, cy;
+  RowRange rows[3];
+  open_block<MULTI, CAP>(b, s0, b.startNext, i0, n, b.keys[il], sc, plan, cx, cy, rows);
   if (CAP > 0 && plan.use) stage(plan, b.x1, tx);
   __syncthreads();
   uint32_t cand = 0;
   if (i < n) {
-    const uint32_t key = b.keys[i];
-    const DevScene sc = scene_of_slot<MULTI>(b, s0, key);
-    const uint32_t local = key - sc.cellBase;
-    const int cy = (int)(local / (uint32_t)sc.nx);
-    const int cx = (int)local - cy * sc.nx;
-    const float2 xi = b.x1[i];
     float d0 = 0.0f, d1 = 0.0f;
     const bool near = wave_near(p, xi);
     if (CAP > 0 && plan.use && near)
-      cand = density_sum<true>(b.startNext, sc, cx, cy, tx, TileIndex(plan), p, xi, d0, d1);
+      cand = density_sum<true>(rows, tx, TileIndex(plan), p, xi, d0, d1);
     else if (near)
-      cand = density_sum<true>(b.startNext, sc, cx, cy, b.x1, SlotIndex(), p, xi, d0, d1);
+      cand = density_sum<true>(rows, b.x1, SlotIndex(), p, xi, d0, d1);
     else
-      cand = density_sum<false>(b.startNext, sc, cx, cy, b.x1, SlotIndex(), p, xi, d0, d1);
+      cand = density_sum<false>(rows, b.x1, SlotIndex(), p, xi, d0, d1);
     b.dens[i] = make_float2(d0, d1);
     b.pres[i] = make_float2(p.k * (d0 - p.rho0), p.kn * d1);  // sph.h:478-481
   }
@@ -1075,12 +1087,11 @@ __global__ __launch_bounds__(kBlock) void k_density(Buffers b, DevParams p, DevS
 // demo4.cpp:239-255 in Jacobi order: -delta_ij/2 from the particle's own visit
 // and +delta_ji/2 from the neighbour's visit (n_ji = -n_ij).
 template <bool NEAR, typename Idx>
-__device__ __forceinline__ void delta_sum(const uint32_t *start, const DevScene &sc, int cx, int cy, const float2 *X,
-                                          const float2 *P, Idx idx, const DevParams &p, float2 xi, float2 pi,
-                                          float &accx, float &accy) {
+__device__ __forceinline__ void delta_sum(const RowRange (&rows)[3], const float2 *X, const float2 *P, Idx idx,
+                                          const DevParams &p, float2 xi, float2 pi, float &accx, float &accy) {
   const float invH = in_vgpr(p.invH), dt2 = in_vgpr(p.dt2);
   for_each_pair(
-      start, sc, cx, cy, X, idx, xi, p.h2,
+      rows, X, idx, xi, p.h2,
       [&](uint32_t j, float Rx, float Ry, float r2, bool use) {
         const float2 pj = P[j];
         float r, inv;
@@ -1106,42 +1117,38 @@ __device__ __forceinline__ void delta_sum(const uint32_t *start, const DevScene 
 template <bool MULTI, int CAP>
 __global__ __launch_bounds__(kBlock) void k_delta(Buffers b, DevParams p, DevScene s0, int n) {
   __shared__ float2 tx[CAP > 0 ? CAP : 1];
-  __shared__ TilePlan plan;
   const int i0 = (int)(blockIdx.x * kBlock);
   const int i = i0 + (int)threadIdx.x;
-  plan_new<MULTI, CAP>(b, s0, i0, n, plan);
-  if (CAP > 0 && plan.use) {
-    stage(plan, b.x1, tx);
-  }
+  const int il = min(i, n - 1);
+  const float2 xi = b.x1[il];
+  const float2 pi = b.pres[il];
+  const float2 pv = b.prev[il];
+  TilePlan plan;
+  DevScene sc;
+  int cx, cy;
+  RowRange rows[3];
+  open_block<MULTI, CAP>(b, s0, b.startNext, i0, n, b.keys[il], sc, plan, cx, cy, rows);
+  if (CAP > 0 && plan.use) stage(plan, b.x1, tx);
   __syncthreads();
   // Lanes past n stay active (collide_wave reduces over the whole wave) but
-  // read and write nothing.
+  // write nothing.
   const bool live = i < n;
-  DevScene sc = s0;
   float x = 0.0f, y = 0.0f;
   if (live) {
-    const uint32_t key = b.keys[i];
-    sc = scene_of_slot<MULTI>(b, s0, key);
-    const uint32_t local = key - sc.cellBase;
-    const int cy = (int)(local / (uint32_t)sc.nx);
-    const int cx = (int)local - cy * sc.nx;
-    const float2 xi = b.x1[i];
-    const float2 pi = b.pres[i];
     float accx = 0.0f, accy = 0.0f;
     const bool near = wave_near(p, xi);
     if (CAP > 0 && plan.use && near)
-      delta_sum<true>(b.startNext, sc, cx, cy, tx, b.pres, TileIndex(plan), p, xi, pi, accx, accy);
+      delta_sum<true>(rows, tx, b.pres, TileIndex(plan), p, xi, pi, accx, accy);
     else if (near)
-      delta_sum<true>(b.startNext, sc, cx, cy, b.x1, b.pres, SlotIndex(), p, xi, pi, accx, accy);
+      delta_sum<true>(rows, b.x1, b.pres, SlotIndex(), p, xi, pi, accx, accy);
     else
-      delta_sum<false>(b.startNext, sc, cx, cy, b.x1, b.pres, SlotIndex(), p, xi, pi, accx, accy);
+      delta_sum<false>(rows, b.x1, b.pres, SlotIndex(), p, xi, pi, accx, accy);
     if (b.dxOut) b.dxOut[i] = make_float2(accx, accy);
     x = accx + xi.x;                                      // demo4.cpp:253
     y = accy + xi.y;
   }
   collide_wave<MULTI>(b, p, sc, x, y, live);              // demo4.cpp:411-444
   if (live) {
-    const float2 pv = b.prev[i];
     b.x0[i] = make_float2(x, y);
     b.v[i] = make_float2((x - pv.x) * p.invDt, (y - pv.y) * p.invDt);  // demo4.cpp:449
   }

@@ -68,3 +68,25 @@ def test_placement_from_its_smallest_step_on():
     spec = _spec(640, 615, 400.0)
     spec.positions[:3000] = (np.array([100.2, 100.2]) + np.random.RandomState(3).uniform(0, 0.6, (3000, 2))).astype(np.float32)
     _check(spec, SPHParams(k=0.0, k_near=0.0, sigma=0.0, beta=0.0), (0.0, -4000.0), [2, 6], caps=(1024, 1024, 1024))
+
+
+@pytest.mark.parametrize("cap", [0, 1024])
+def test_workgroups_across_scenes_and_past_the_binned_particles(cap):
+    # scenes of 1 to 600 particles: 256-slot workgroups within one scene, across several, and partly filled;
+    # then particles added past the binned ones
+    specs = []
+    for s, n in enumerate([1, 2, 600, 255, 257, 3, 512, 31, 64, 400]):
+        cols = int(np.ceil(np.sqrt(n)))
+        spec = _spec(cols, cols, 2.0 * (cols // 2 + 4), seed=50 + s, limit=n)
+        specs.append(spec)
+    sim, ref = gpu_for(specs, SPHParams(sigma=0.2), (0.0, -9.8)), oracle_for(specs, SPHParams(sigma=0.2), gravity=(0.0, -9.8))
+    sim.set_tuning(autotune=False, tile_cap=(cap,) * 3, wide_max_particles=0)
+    for m in (1, 4):
+        sim.Update(DT, m)
+        ref.step(DT, m)
+        assert_bit_exact(sim.get_state(), ref.state(), f"{m}: ")
+        for k in range(2):
+            sim.AddParticle((0.3 * k, 0.2 * m), scene=2)
+            ref.add_particles(2, np.array([[0.3 * k, 0.2 * m]], np.float32))
+    sim.close()
+    ref.close()
