@@ -51,42 +51,6 @@ __device__ __forceinline__ void length_of(bool near, float r2, float &r, float &
 }
 __device__ __forceinline__ float root_of(bool near, float r2) { return near ? near_sqrt(r2) : pair_sqrt(r2); }
 
-// What a workgroup's pair walk starts from: the tile plan of its slots
-// [i0, min(i0 + kBlock, end)), whose first and last cell bound the others', and
-// the calling particle's scene, cell and rows (key: its cell).  Every wave
-// plans for itself in scalar registers, so the plan needs no barrier, and the
-// particle's rows are requested before the tile is staged: keys, cell starts
-// and tile are three memory round trips, where a plan left in LDS by one thread
-// and rows read after the tile took five.  A slot range within one scene reads
-// that scene once.  96 scenes, 1.76 M particles: viscosity 66.6 -> 62.5 us,
-// density 45.2 -> 41.9, delta 61.5 -> 60; one scene of 1,048,576: unchanged
-// (its kernels are bound by the walk's issue: of 38.5 us viscosity, 17 remain
-// without the walk, 25 with the walk's tests alone).
-template <bool MULTI, int CAP>
-__device__ __forceinline__ void open_block(const Buffers &b, const DevScene &s0, const uint32_t *start, int i0,
-                                           int end, uint32_t key, DevScene &sc, TilePlan &plan, int &cx, int &cy,
-                                           RowRange (&rows)[3]) {
-  const uint32_t kA = (uint32_t)__builtin_amdgcn_readfirstlane((int)b.keys[i0]);
-  const uint32_t kB = (uint32_t)__builtin_amdgcn_readfirstlane((int)b.keys[min(i0 + kBlock, end) - 1]);
-  if (MULTI) {
-    const int a = __builtin_amdgcn_readfirstlane(scene_index(b, kA));
-    const int e = __builtin_amdgcn_readfirstlane(scene_index(b, kB));
-    sc = b.scenes[a];
-    plan_tile<CAP>(start, sc, kA, kB, plan);
-    if (a != e) {
-      plan.use = 0;
-      sc = b.scenes[scene_index(b, key)];
-    }
-  } else {
-    sc = s0;
-    plan_tile<CAP>(start, sc, kA, kB, plan);
-  }
-  const uint32_t local = key - sc.cellBase;
-  cy = (int)(local / (uint32_t)sc.nx);
-  cx = (int)local - cy * sc.nx;
-  row_ranges(start, sc, cx, cy, rows);
-}
-
 // For every candidate slot j (of the three row ranges) of the particle at xi whose
 // r2 < h2 (sph.h:470, 488, 502), in candidate order, applies the pair's
 // contribution: apply(term(j, Rx, Ry, r2, true)).  term(..., false) must return
@@ -393,7 +357,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_predict(Buffers b, DevParams p,
   int pcx = -2, pcy = -2;  // cell of the last binning (none: not adjacent to any cell)
   RowRange rows[3];
   if (tileVisc) {
-    open_block<MULTI, CAP>(b, s0, b.startCur, i0, nBinned, b.keys[min(i, nBinned - 1)], sc, plan, pcx, pcy, rows);
+    open_block<MULTI, CAP, kBlock>(b, s0, b.startCur, i0, nBinned, b.keys[min(i, nBinned - 1)], sc, plan, pcx, pcy, rows);
     if (CAP > 0 && plan.use) stage(plan, b.x0, tx);
     __syncthreads();
   } else if (MULTI && binned) {
@@ -1055,7 +1019,7 @@ __global__ __launch_bounds__(kBlock) void k_density(Buffers b, DevParams p, DevS
   DevScene sc;
   int cx, cy;
   RowRange rows[3];
-  open_block<MULTI, CAP>(b, s0, b.startNext, i0, n, b.keys[il], sc, plan, cx, cy, rows);
+  open_block<MULTI, CAP, kBlock>(b, s0, b.startNext, i0, n, b.keys[il], sc, plan, cx, cy, rows);
   if (CAP > 0 && plan.use) stage(plan, b.x1, tx);
   __syncthreads();
   uint32_t cand = 0;
@@ -1127,7 +1091,7 @@ __global__ __launch_bounds__(kBlock) void k_delta(Buffers b, DevParams p, DevSce
   DevScene sc;
   int cx, cy;
   RowRange rows[3];
-  open_block<MULTI, CAP>(b, s0, b.startNext, i0, n, b.keys[il], sc, plan, cx, cy, rows);
+  open_block<MULTI, CAP, kBlock>(b, s0, b.startNext, i0, n, b.keys[il], sc, plan, cx, cy, rows);
   if (CAP > 0 && plan.use) stage(plan, b.x1, tx);
   __syncthreads();
   // Lanes past n stay active (collide_wave reduces over the whole wave) but

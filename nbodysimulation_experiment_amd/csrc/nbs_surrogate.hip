@@ -151,8 +151,6 @@ constexpr int kPoolBytes = kHeadBytes > kStageBytes ? kHeadBytes : kStageBytes;
 
 // Per-particle inputs of the pair layer.
 struct PartInfo {
-  DevScene sc;
-  int cx, cy;
   float2 xi;
   float vix, viy;
   float fr, fn;  // normalised density, near density
@@ -166,14 +164,8 @@ struct PartRaw {
 };
 __device__ __forceinline__ PartRaw part_raw(const Buffers &b, int i) { return {b.keys[i], b.x1[i], b.prev[i], b.dens[i]}; }
 
-template <bool MULTI>
-__device__ __forceinline__ PartInfo part_info(const Buffers &b, const DevParams &p, const DevScene &s0,
-                                              const float *norm, const PartRaw &r) {
+__device__ __forceinline__ PartInfo part_info(const DevParams &p, const float *norm, const PartRaw &r) {
   PartInfo q;
-  q.sc = scene_of_slot<MULTI>(b, s0, r.key);
-  const uint32_t local = r.key - q.sc.cellBase;
-  q.cy = (int)(local / (uint32_t)q.sc.nx);
-  q.cx = (int)local - q.cy * q.sc.nx;
   q.xi = r.x;
   q.vix = (q.xi.x - r.pv.x) * p.invDt;
   q.viy = (q.xi.y - r.pv.y) * p.invDt;
@@ -193,6 +185,7 @@ struct Cursor {
   // rows tested up front (cursor_rows): the masks and source bases of the
   // rows after the current one
   uint32_t m1, b1, m2, b2;
+  RowRange r0, r1, r2;  // the rows not walked yet
 };
 
 // Neighbour data of a wave's candidates: an LDS copy of the three candidate
@@ -210,14 +203,14 @@ struct PairSrc {
   }
 };
 
-__device__ __forceinline__ bool cursor_next_row(Cursor &cu, const uint32_t *start, const PartInfo &q,
-                                                const PairSrc &src) {
+__device__ __forceinline__ bool cursor_next_row(Cursor &cu, const PairSrc &src) {
   while (cu.d < 3) {
-    const RowRange rr = row_range(start, q.sc, q.cx, q.cy, cu.d - 1);
     const int r = cu.d++;
-    if (rr.j0 < rr.j1) {
-      cu.j = rr.j0;
-      cu.jend = rr.j1;
+    cu.j = cu.r0.j0;
+    cu.jend = cu.r0.j1;
+    cu.r0 = cu.r1;
+    cu.r1 = cu.r2;
+    if (cu.j < cu.jend) {
       cu.tb = src.base(r);
       return true;
     }
@@ -225,17 +218,8 @@ __device__ __forceinline__ bool cursor_next_row(Cursor &cu, const uint32_t *star
   return false;
 }
 
-// Plans the wave's tile and stages it when it fits (every lane must call it).
-template <bool MULTI>
-__device__ __forceinline__ PairSrc stage_pairs(const Buffers &b, const DevScene &s0, int base, int n,
-                                               unsigned char *pool, TilePlan &plan) {
-  if (threadIdx.x == 0) {
-    const uint32_t kA = b.keys[base], kB = b.keys[min(base + kWaveRows, n) - 1];
-    const DevScene sa = scene_of_slot<MULTI>(b, s0, kA);
-    plan_tile<kTileCap>(b.startNext, sa, kA, kB, plan);
-    if (MULTI && sa.cellBase != scene_of_slot<MULTI>(b, s0, kB).cellBase) plan.use = 0;
-  }
-  __syncthreads();
+// Stages the planned tile when it fits (every lane must call it).
+__device__ __forceinline__ PairSrc stage_pairs(const Buffers &b, const TilePlan &plan, unsigned char *pool) {
   PairSrc src;
   src.tiled = plan.use != 0;
   src.rowStart0 = plan.rowStart[0], src.rowStart1 = plan.rowStart[1], src.rowStart2 = plan.rowStart[2];
@@ -320,6 +304,7 @@ constexpr uint32_t kWalkRowMax = 32;
 __device__ __forceinline__ bool rows_fit(const RowRange (&rows)[3], bool live) {
   bool fit = true;
   if (live)
+#pragma unroll
     for (int d = 0; d < 3; ++d) fit = fit && rows[d].j1 - rows[d].j0 <= kWalkRowMax;
   return __ballot(!fit) == 0ull;
 }
@@ -349,9 +334,8 @@ __device__ __forceinline__ void cursor_rows(Cursor &cu, const RowRange (&rows)[3
 // into a mask, whose bits are then taken lowest first (candidate order); with
 // rows (the cursor loaded by cursor_rows) the masks of all three rows are
 // there already.
-__device__ __forceinline__ bool next_pair(Cursor &cu, const Buffers &b, const DevParams &p, const PairSrc &src,
-                                          const PartInfo &q, int i, bool rows, uint32_t &t, float2 &xj, float &Rx,
-                                          float &Ry, float &r2) {
+__device__ __forceinline__ bool next_pair(Cursor &cu, const DevParams &p, const PairSrc &src, const PartInfo &q, int i,
+                                          bool rows, uint32_t &t, float2 &xj, float &Rx, float &Ry, float &r2) {
   for (;;) {
     if (cu.mask) {
       const uint32_t bit = (uint32_t)__builtin_ctz(cu.mask);
@@ -374,7 +358,7 @@ __device__ __forceinline__ bool next_pair(Cursor &cu, const Buffers &b, const De
       cu.m2 = 0u;
       continue;
     }
-    if (cu.j >= cu.jend && !cursor_next_row(cu, b.startNext, q, src)) {
+    if (cu.j >= cu.jend && !cursor_next_row(cu, src)) {
       cu.done = true;
       return false;
     }
@@ -419,20 +403,19 @@ __device__ __forceinline__ W1Operands load_w1(const uint16_t *w1b) {
 // A operands (K = 16) of the two row tiles from each lane's own feature words:
 // tile 0 rows are lanes 0..31, tile 1 rows lanes 32..63; lane (c, g) supplies
 // features 8g .. 8g + 7 of its row, so one half of each tile's words crosses
-// the lane halves (words 6, 7 are zero).
+// the lane halves (words 6, 7 are zero): one exchange per word (with shuffles
+// through the LDS unit the 262,144-particle forward took 62 us instead of 60).
 struct PairA {
   bf16x8 t0, t1;
 };
 
 __device__ __forceinline__ PairA pair_operands(const uint32_t w[8]) {
-  const int g = (threadIdx.x >> 5) & 1;
-  const uint32_t s0 = g ? w[0] : w[4], s1 = g ? w[1] : w[5], s2 = g ? w[2] : 0u, s3 = g ? w[3] : 0u;
-  const uint32_t r0 = (uint32_t)__shfl_xor((int)s0, 32, 64), r1 = (uint32_t)__shfl_xor((int)s1, 32, 64);
-  const uint32_t r2 = (uint32_t)__shfl_xor((int)s2, 32, 64), r3 = (uint32_t)__shfl_xor((int)s3, 32, 64);
-  PairA a;
-  a.t0 = g ? bf8(r0, r1, r2, r3) : bf8(w[0], w[1], w[2], w[3]);
-  a.t1 = g ? bf8(w[4], w[5], 0u, 0u) : bf8(r0, r1, r2, r3);
-  return a;
+  // swap(x, y): y's lower half moves to x's upper half and back
+  const auto r0 = __builtin_amdgcn_permlane32_swap(w[0], w[4], false, false);
+  const auto r1 = __builtin_amdgcn_permlane32_swap(w[1], w[5], false, false);
+  const auto r2 = __builtin_amdgcn_permlane32_swap(w[2], 0u, false, false);
+  const auto r3 = __builtin_amdgcn_permlane32_swap(w[3], 0u, false, false);
+  return {bf8(r0[0], r1[0], r2[0], r3[0]), bf8(r0[1], r1[1], r2[1], r3[1])};
 }
 
 // Pre-activations z = F W1^T of one row tile (C layout, lane = hidden unit).
@@ -481,13 +464,110 @@ __device__ __forceinline__ void store_tile_f32(float4 *dst, int lane, const floa
   for (int q = 0; q < 8; ++q) dst[q * 64 + lane] = make_float4(lo[2 * q], hi[2 * q], lo[2 * q + 1], hi[2 * q + 1]);
 }
 
+// Operands (K = hidden) of a half of a tile whose C layout has the particle as
+// its lane: k_order on packed BF16 words.
+__device__ __forceinline__ void k_operands(const floatx16 &z, bf16x8 &op0, bf16x8 &op1) {
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int r = 8 * s;
+    const auto a = __builtin_amdgcn_permlane32_swap(pack2(z[r], z[r + 1]), pack2(z[r + 4], z[r + 5]), false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(pack2(z[r + 2], z[r + 3]), pack2(z[r + 6], z[r + 7]), false, false);
+    (s ? op1 : op0) = bf8(a[0], b[0], a[1], b[1]);
+  }
+}
+
+// Registers of a C-layout tile from a vector indexed by its row: v[c_row(r, g)].
+__device__ __forceinline__ floatx16 by_row(const float *v) {
+  floatx16 z;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float4 f = *reinterpret_cast<const float4 *>(v + 8 * q + 4 * ((threadIdx.x >> 5) & 1));
+    z[4 * q] = f.x, z[4 * q + 1] = f.y, z[4 * q + 2] = f.z, z[4 * q + 3] = f.w;
+  }
+  return z;
+}
+
+// The head without LDS, for a forward that keeps no activations.  The pair sums
+// h[tile][hidden half] have the particle as their lane (column) and the hidden
+// units in their registers, so that a layer's packed outputs are, after one
+// exchange between the wave's halves, the next layer's operands, both row tiles
+// share the weights' operands, and lane l ends with all 64 values of G of
+// particle l for the output layer's FP32 sum (k ascending, as the training
+// forward adds them from LDS: the same products in the same order).  262,144
+// particles: one tile after the other through LDS 20 of the forward's 60 us,
+// all of it 46 us now.
+__device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_t np, const SurrogateBufs &m) {
+  const float *prm = m.params;
+  const auto cnt = __builtin_amdgcn_permlane32_swap(__float_as_uint((float)np), __float_as_uint((float)np), false, false);
+  bf16x8 op[2][4], om[2][4];  // H, M: tile, K step
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) k_operands(h[t][y], op[t][2 * y], op[t][2 * y + 1]);
+  // output half y of a layer for both tiles
+  auto dense = [&](const uint16_t *W, int y, const bf16x8 (&in)[2][4], floatx16 &z0, floatx16 &z1) {
+    z0 = zero16(), z1 = zero16();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const bf16x8 w = load_wb16(W, kHid, 32 * y, 16 * s);
+      z0 = mfma16(w, in[0][s], z0);
+      z1 = mfma16(w, in[1][s], z1);
+    }
+  };
+  // M = W2 H + n b2, kept as BF16
+#pragma unroll
+  for (int y = 0; y < 2; ++y) {
+    floatx16 z0, z1;
+    dense(m.w2b, y, op, z0, z1);
+    const floatx16 b2 = by_row(prm + kOffB2 + 32 * y);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      z0[r] += __uint_as_float(cnt[0]) * b2[r];
+      z1[r] += __uint_as_float(cnt[1]) * b2[r];
+    }
+    k_operands(z0, om[0][2 * y], om[0][2 * y + 1]);
+    k_operands(z1, om[1][2 * y], om[1][2 * y + 1]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // G = relu(W3 M + b3), FP32; then o = W4 G + b4
+  float2 o = make_float2(prm[kOffB4], prm[kOffB4 + 1]);
+#pragma unroll
+  for (int y = 0; y < 2; ++y) {
+    floatx16 z0, z1;
+    dense(m.w3b, y, om, z0, z1);
+    const floatx16 b3 = by_row(prm + kOffB3 + 32 * y);
+    floatx16 g[2];  // rows c_row(r, 0), c_row(r, 1) of the lane's own particle
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(relu(z0[r] + b3[r])),
+                                                      __float_as_uint(relu(z1[r] + b3[r])), false, false);
+      g[0][r] = __uint_as_float(q[0]);
+      g[1][r] = __uint_as_float(q[1]);
+    }
+#pragma unroll
+    for (int k = 0; k < 32; ++k) {
+      const float v = g[(k >> 2) & 1][4 * (k >> 3) + (k & 3)];
+      o.x = __builtin_fmaf(prm[kOffW4 + 32 * y + k], v, o.x);
+      o.y = __builtin_fmaf(prm[kOffW4 + kHid + 32 * y + k], v, o.y);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+v"(o.x), "+v"(o.y));  // a half of W4 in scalar registers at a time: both would spill
+  }
+  return o;
+}
+
+// One wave takes 64 particles; every iteration of the walk adds one pair of each
+// through the matrix cores.  Bound by the issue of an iteration's about 180
+// vector instructions (relu and packing 64, features 40; its 12 products take
+// two thirds of that time beside them) and by the start of each wave's walk.
+// Two waves per SIMD: for three the compiler spills inside the walk (80 us at
+// 262,144 particles, 46 without).
 template <bool MULTI, bool TRAIN>
-__global__ __launch_bounds__(64, TRAIN ? 2 : 3) void k_sur_forward(Buffers b, DevParams p, DevScene s0, int n, SurrogateBufs m,
-                                                    int mode) {
+__global__ __launch_bounds__(64, 2) void k_sur_forward(Buffers b, DevParams p, DevScene s0, int n, SurrogateBufs m,
+                                                       int mode) {
   // LDS: the staged candidates during the pair layer, then the head's operand
   // rows (hb: H, then M, of one row tile as BF16) and G (FP32)
   __shared__ __align__(16) unsigned char pool[kPoolBytes];
-  __shared__ TilePlan plan;
   __shared__ float shCnt[kWaveRows];
   uint16_t(*hb)[kHbStride] = reinterpret_cast<uint16_t(*)[kHbStride]>(pool);
   float(*gbuf)[kGStride] = reinterpret_cast<float(*)[kGStride]>(pool + kHbBytes);
@@ -499,32 +579,34 @@ __global__ __launch_bounds__(64, TRAIN ? 2 : 3) void k_sur_forward(Buffers b, De
   const W1Operands w1 = load_w1(m.w1b);
   const bf16x8 sel[2] = {selection(0), selection(1)};
   const PartRaw raw = part_raw(b, min(me, n - 1));  // a lane past n reads the last particle, unused
-  const PairSrc src = stage_pairs<MULTI>(b, s0, base, n, pool, plan);
+  TilePlan plan;
+  DevScene scMe;
+  int cx, cy;
+  RowRange rr[3];
+  open_block<MULTI, kTileCap, kWaveRows>(b, s0, b.startNext, base, n, raw.key, scMe, plan, cx, cy, rr);
+  const PairSrc src = stage_pairs(b, plan, pool);
 
   // 1. pair layer: H_i = sum_j relu(W1 f_ij), each term rounded to BF16
-  PartInfo q{};
-  Cursor cu{0u, 0u, 0u, 0, true, 0u, 0u};
-  if (me < n) {
-    q = part_info<MULTI>(b, p, s0, norm, raw);
-    cu.done = false;
-  }
-  floatx16 h00 = zero16(), h01 = zero16(), h10 = zero16(), h11 = zero16();  // tile, hidden half
+  const PartInfo q = part_info(p, norm, raw);
+  Cursor cu{0u, 0u, 0u, 0, me >= n, 0u, 0u, 0u, 0u, 0u, 0u, rr[0], rr[1], rr[2]};
+  floatx16 h[2][2] = {{zero16(), zero16()}, {zero16(), zero16()}};  // tile, hidden half
+  // the training forward keeps the particle in the rows, the other in the lanes
+  auto add = [&](bf16x8 z, int s, floatx16 &acc) { acc = TRAIN ? mfma16(sel[s], z, acc) : mfma16(z, sel[s], acc); };
+  auto add_tile = [&](bf16x8 a, floatx16 (&acc)[2]) {
+    floatx16 zlo, zhi;
+    pair_layer(a, w1, zlo, zhi);
+    add(relu_rows(zlo, 0), 0, acc[0]);  // K steps 0 and 1 of each hidden half
+    add(relu_rows(zhi, 0), 0, acc[1]);
+    add(relu_rows(zlo, 1), 1, acc[0]);
+    add(relu_rows(zhi, 1), 1, acc[1]);
+  };
   uint32_t np = 0;
-  auto pair_pass = [&](const PairSrc &sp) {
-    // rows up front except for the multi-scene training forward, where they
-    // measured slower
-    bool rows = false;
-    if (!(MULTI && TRAIN)) {
-      RowRange rr[3] = {};
-      if (me < n) row_ranges(b.startNext, q.sc, q.cx, q.cy, rr);  // the six cell starts in flight together
-      rows = rows_fit(rr, me < n);
-      if (rows && me < n) cursor_rows(cu, rr, p, sp, q, me);
-    }
+  auto walk = [&](const PairSrc &sp, auto rows) {
     for (;;) {
       uint32_t t = 0;
       float2 xj = make_float2(0.0f, 0.0f);
       float Rx = 0.0f, Ry = 0.0f, r2 = 0.0f;
-      const bool have = next_pair(cu, b, p, sp, q, me, rows, t, xj, Rx, Ry, r2);
+      const bool have = next_pair(cu, p, sp, q, me, rows(), t, xj, Rx, Ry, r2);
       if (__ballot(have) == 0ull) break;  // wave-uniform
       uint32_t w[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
       if (have) {
@@ -532,33 +614,65 @@ __global__ __launch_bounds__(64, TRAIN ? 2 : 3) void k_sur_forward(Buffers b, De
         ++np;
       }
       const PairA a = pair_operands(w);
-      floatx16 zlo, zhi;
-      // K steps 0 and 1 of each tile and hidden half
-      pair_layer(a.t0, w1, zlo, zhi);
-      h00 = mfma16(sel[0], relu_rows(zlo, 0), h00);
-      h01 = mfma16(sel[0], relu_rows(zhi, 0), h01);
-      h00 = mfma16(sel[1], relu_rows(zlo, 1), h00);
-      h01 = mfma16(sel[1], relu_rows(zhi, 1), h01);
-      pair_layer(a.t1, w1, zlo, zhi);
-      h10 = mfma16(sel[0], relu_rows(zlo, 0), h10);
-      h11 = mfma16(sel[0], relu_rows(zhi, 0), h11);
-      h10 = mfma16(sel[1], relu_rows(zlo, 1), h10);
-      h11 = mfma16(sel[1], relu_rows(zhi, 1), h11);
+      add_tile(a.t0, h[0]);
+      add_tile(a.t1, h[1]);
     }
   };
-  // one copy of the pass per source, so that the tile's loads are LDS loads
-  // (a pointer that may be either is a flat address)
+  // One copy of the walk per source, so that the tile's loads are LDS loads (a
+  // pointer that may be either is a flat address), and per kind of walk: their
+  // cursors hold different registers.
+  auto pair_pass = [&](const PairSrc &sp) {
+    if (rows_fit(rr, me < n)) {
+      if (me < n) cursor_rows(cu, rr, p, sp, q, me);
+      walk(sp, std::true_type());
+    } else {
+      walk(sp, std::false_type());
+    }
+  };
   if (src.tiled)
     pair_pass(tile_src(src, pool));
   else
     pair_pass(slot_src(src, b));
-  shCnt[lane] = (float)np;
-  if (m.pairPart) {
+  auto pair_total = [&] {
+    if (!m.pairPart) return;
     uint32_t tot = np;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) tot += (uint32_t)__shfl_xor((int)tot, off, 64);
     if (lane == 0) m.pairPart[blockIdx.x] = tot;
+  };
+  // o of particle i: the network's output, and the state after the relaxation
+  // and the boundary collisions
+  auto finish = [&](int i, bool live, float2 o) {
+    if (live && m.out) reinterpret_cast<float2 *>(m.out)[i] = o;
+    if (!(mode & kFwdState)) return;
+    DevScene sc = s0;
+    float x = 0.0f, y = 0.0f;
+    if (live) {
+      sc = scene_of_slot<MULTI>(b, s0, b.keys[i]);
+      const float2 xi = b.x1[i];
+      x = xi.x + o.x * norm[5];
+      y = xi.y + o.y * norm[5];
+    }
+    collide_wave<MULTI>(b, p, sc, x, y, live);                                 // demo4.cpp:411-444
+    if (live) {
+      if (mode & kFwdPressure) {
+        const float2 d = b.dens[i];
+        b.pres[i] = make_float2(p.k * (d.x - p.rho0), p.kn * d.y);             // sph.h:478-481
+      }
+      const float2 pv = b.prev[i];
+      b.x0[i] = make_float2(x, y);
+      b.v[i] = make_float2((x - pv.x) * p.invDt, (y - pv.y) * p.invDt);        // demo4.cpp:446-450
+    }
+  };
+  if constexpr (!TRAIN) {
+    const float2 o = head_output(h, np, m);
+    pair_total();
+    finish(me, me < n, o);
+    return;
   }
+  // (TRAIN from here on)
+  pair_total();
+  shCnt[lane] = (float)np;
 
   // 2. head, one 32-row tile at a time: C = A W^T with A in hb (BF16)
   auto dense = [&](const uint16_t *W, floatx16 &olo, floatx16 &ohi) {
@@ -575,8 +689,8 @@ __global__ __launch_bounds__(64, TRAIN ? 2 : 3) void k_sur_forward(Buffers b, De
   };
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
-    const floatx16 &hlo = t ? h10 : h00;
-    const floatx16 &hhi = t ? h11 : h01;
+    const floatx16 &hlo = h[t][0];
+    const floatx16 &hhi = h[t][1];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
@@ -623,31 +737,7 @@ __global__ __launch_bounds__(64, TRAIN ? 2 : 3) void k_sur_forward(Buffers b, De
     float o = prm[kOffB4 + g];
     for (int k = 0; k < kHid; ++k) o = __builtin_fmaf(prm[kOffW4 + g * kHid + k], gbuf[c][k], o);
     const float oy = __shfl_down(o, 32, 64);
-    const bool head = g == 0 && i < n;
-    if (head && m.out) {
-      m.out[2 * (size_t)i] = o;
-      m.out[2 * (size_t)i + 1] = oy;
-    }
-    if (mode & kFwdState) {
-      DevScene sc = s0;
-      float x = 0.0f, y = 0.0f;
-      if (head) {
-        sc = scene_of_slot<MULTI>(b, s0, b.keys[i]);
-        const float2 xi = b.x1[i];
-        x = xi.x + o * norm[5];
-        y = xi.y + oy * norm[5];
-      }
-      collide_wave<MULTI>(b, p, sc, x, y, head);                               // demo4.cpp:411-444
-      if (head) {
-        if (mode & kFwdPressure) {
-          const float2 d = b.dens[i];
-          b.pres[i] = make_float2(p.k * (d.x - p.rho0), p.kn * d.y);           // sph.h:478-481
-        }
-        const float2 pv = b.prev[i];
-        b.x0[i] = make_float2(x, y);
-        b.v[i] = make_float2((x - pv.x) * p.invDt, (y - pv.y) * p.invDt);      // demo4.cpp:446-450
-      }
-    }
+    finish(i, g == 0 && i < n, make_float2(o, oy));
   }
 }
 
@@ -952,7 +1042,6 @@ __global__ __launch_bounds__(64) void k_sur_back_pairs(Buffers b, DevParams p, D
                                                      float *pairPart) {
   __shared__ uint32_t fw[kWaveRows][kFeat / 2];
   __shared__ __align__(16) unsigned char pool[kStageBytes];
-  __shared__ TilePlan plan;
   const int lane = threadIdx.x, c = lane & 31, g = lane >> 5;
   const float *norm = m.params + kOffNorm;
   const W1Operands w1 = load_w1(m.w1b);
@@ -961,7 +1050,12 @@ __global__ __launch_bounds__(64) void k_sur_back_pairs(Buffers b, DevParams p, D
     const int me = base + lane;
     __syncthreads();  // the previous group's tile is no longer read
     const PartRaw raw = part_raw(b, min(me, n - 1));  // a lane past n reads the last particle, unused
-    const PairSrc src = stage_pairs<MULTI>(b, s0, base, n, pool, plan);
+    TilePlan plan;
+    DevScene sc;
+    int cx, cy;
+    RowRange rr[3];
+    open_block<MULTI, kTileCap, kWaveRows>(b, s0, b.startNext, base, n, raw.key, sc, plan, cx, cy, rr);
+    const PairSrc src = stage_pairs(b, plan, pool);
     // dH of the rows this lane's accumulator registers hold (the second tile
     // may lie past the last particle: its lanes have no pairs)
     floatx16 d00, d01, d10, d11;  // tile, hidden half
@@ -973,17 +1067,13 @@ __global__ __launch_bounds__(64) void k_sur_back_pairs(Buffers b, DevParams p, D
       d00[2 * k] = u.x, d01[2 * k] = u.y, d00[2 * k + 1] = u.z, d01[2 * k + 1] = u.w;
       d10[2 * k] = v.x, d11[2 * k] = v.y, d10[2 * k + 1] = v.z, d11[2 * k + 1] = v.w;
     }
-    PartInfo q{};
-    Cursor cu{0u, 0u, 0u, 0, true, 0u, 0u};
-    if (me < n) {
-      q = part_info<MULTI>(b, p, s0, norm, raw);
-      cu.done = false;
-    }
+    const PartInfo q = part_info(p, norm, raw);
+    Cursor cu{0u, 0u, 0u, 0, me >= n, 0u, 0u, 0u, 0u, 0u, 0u, rr[0], rr[1], rr[2]};
     for (;;) {
       uint32_t t = 0;
       float2 xj = make_float2(0.0f, 0.0f);
       float Rx = 0.0f, Ry = 0.0f, r2 = 0.0f;
-      const bool have = next_pair(cu, b, p, src, q, me, false, t, xj, Rx, Ry, r2);
+      const bool have = next_pair(cu, p, src, q, me, false, t, xj, Rx, Ry, r2);
       if (__ballot(have) == 0ull) break;  // wave-uniform
       uint32_t w[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
       if (have) pair_words(w, src, p, norm, q, t, xj, Rx, Ry, r2);

@@ -23,3 +23,27 @@ def test_gradient_at_block_edges(n, cols):
         sim.surrogate_init(3)
         sim.surrogate_calibrate(DT)
         check_frame(sim)
+
+
+@pytest.mark.parametrize("sizes,spacing", [((1,), 0.5), ((33,), 0.5), ((64,), 0.5), ((97, 2, 64, 31), 0.5),
+                                           ((700,), 0.12), ((130, 400), 0.12), ((1500,), 0.05)])
+def test_inference_and_training_forward_agree(sizes, spacing):
+    # the two forms of the head add the same products in the same order: bit-equal states, for partial row
+    # tiles, rows of more than 32 candidates and more candidates than the tile holds
+    states = []
+    for lr in (0.0, 1e-3):
+        specs = []
+        for k, n in enumerate(sizes):
+            cols = int(np.ceil(np.sqrt(n)))
+            pos = volume_positions((0.1, 0.2), cols, cols, spacing, 1.0, seed=n + k, limit=n)
+            specs.append(SceneSpec(30.0, 24.0, 1.0, pos, planes=wall_planes(30.0, 24.0), circles=[(3.0, 3.0, 1.5)]))
+        with ParticleSimulation.from_scenes(specs, SPHParams(k=1e-4, k_near=1e-4), GRAVITY) as sim:
+            sim.surrogate_init(7)
+            sim.surrogate_calibrate(DT)
+            sim.surrogate_set_online_training(lr)
+            sim.surrogate_set_mode(True, 1, 1e30)
+            sim.Update(DT, 1)
+            assert sim.surrogate_report()["fallbacks"] == 0
+            states.append(sim.get_state())
+    for k in ("x", "v", "density"):
+        assert np.array_equal(states[0][k].view(np.uint32), states[1][k].view(np.uint32)), k
