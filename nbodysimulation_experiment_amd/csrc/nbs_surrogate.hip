@@ -140,6 +140,18 @@ __device__ __forceinline__ bf16x8 selection(int s) {
   return bf8(w[0], w[1], w[2], w[3]);
 }
 
+// B operand (K = 16) of the 16 x 32 matrix with ones where k == n.
+__device__ __forceinline__ bf16x8 identity16() {
+  const int c = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
+  uint32_t w[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int k = 8 * g + 2 * q;
+    w[q] = k == c ? 0x3F80u : (k + 1 == c ? 0x3F800000u : 0u);  // BF16 1.0
+  }
+  return bf8(w[0], w[1], w[2], w[3]);
+}
+
 constexpr int kWaveRows = 64;    // particles per wave in the pair kernels
 constexpr int kHbStride = 68;    // BF16 per row of the head operand buffer (padded)
 constexpr int kGStride = kHid + 1;
@@ -372,6 +384,28 @@ __device__ __forceinline__ bool next_pair(Cursor &cu, const DevParams &p, const 
     cu.mask = m;
     cu.j += cnt;
   }
+}
+
+// Runs walk(source, whether the rows were tested up front).  One copy of the
+// walk per source, so that the tile's loads are LDS loads (a pointer that may be
+// either is a flat address), and per kind of walk: their cursors hold different
+// registers.
+template <typename Walk>
+__device__ __forceinline__ void pair_pass(const PairSrc &src, unsigned char *pool, const Buffers &b, const DevParams &p,
+                                          const PartInfo &q, const RowRange (&rr)[3], int i, int n, Cursor &cu,
+                                          Walk &&walk) {
+  auto pass = [&](const PairSrc &sp) {
+    if (rows_fit(rr, i < n)) {
+      if (i < n) cursor_rows(cu, rr, p, sp, q, i);
+      walk(sp, std::true_type());
+    } else {
+      walk(sp, std::false_type());
+    }
+  };
+  if (src.tiled)
+    pass(tile_src(src, pool));
+  else
+    pass(slot_src(src, b));
 }
 
 // The pair's 16 BF16 features as 8 words (features 2k, 2k+1 in word k).
@@ -618,21 +652,7 @@ __global__ __launch_bounds__(64, 2) void k_sur_forward(Buffers b, DevParams p, D
       add_tile(a.t1, h[1]);
     }
   };
-  // One copy of the walk per source, so that the tile's loads are LDS loads (a
-  // pointer that may be either is a flat address), and per kind of walk: their
-  // cursors hold different registers.
-  auto pair_pass = [&](const PairSrc &sp) {
-    if (rows_fit(rr, me < n)) {
-      if (me < n) cursor_rows(cu, rr, p, sp, q, me);
-      walk(sp, std::true_type());
-    } else {
-      walk(sp, std::false_type());
-    }
-  };
-  if (src.tiled)
-    pair_pass(tile_src(src, pool));
-  else
-    pair_pass(slot_src(src, b));
+  pair_pass(src, pool, b, p, q, rr, me, n, cu, walk);
   auto pair_total = [&] {
     if (!m.pairPart) return;
     uint32_t tot = np;
@@ -1034,17 +1054,20 @@ __global__ __launch_bounds__(kUpdateBlock) void k_grad_update(const float *pairP
 // forward pass.  For row tile t the pair layer's pre-activations (C layout:
 // lane = hidden unit, register r = tile row c_row(r, g)), masked and scaled by
 // the rows' dH, are the A operand (hidden x 16 rows) of K step s (registers
-// 8s .. 8s + 7); the same rows' features, staged in LDS, are the B operand
-// (16 rows x 32 features, 16 used).  Each wave accumulates over its particles
-// and writes one 64 x 16 partial.
+// 8s .. 8s + 7); the same rows' features are the B operand (16 rows x 32
+// features, 16 used): the features times the identity, on the matrix core, have
+// the pre-activations' layout, so they need no transposition through LDS (by 16
+// words read per tile and lane and taken apart, a 327,680-particle launch took
+// 135 us instead of 63).  Each wave accumulates over its particles and writes
+// one 64 x 16 partial.
 template <bool MULTI>
-__global__ __launch_bounds__(64) void k_sur_back_pairs(Buffers b, DevParams p, DevScene s0, int n, SurrogateBufs m,
-                                                     float *pairPart) {
-  __shared__ uint32_t fw[kWaveRows][kFeat / 2];
+__global__ __launch_bounds__(64, 2) void k_sur_back_pairs(Buffers b, DevParams p, DevScene s0, int n, SurrogateBufs m,
+                                                          float *pairPart) {
   __shared__ __align__(16) unsigned char pool[kStageBytes];
   const int lane = threadIdx.x, c = lane & 31, g = lane >> 5;
   const float *norm = m.params + kOffNorm;
   const W1Operands w1 = load_w1(m.w1b);
+  const bf16x8 unit = identity16();
   floatx16 glo = zero16(), ghi = zero16();
   for (int base = (int)blockIdx.x * kWaveRows; base < n; base += (int)gridDim.x * kWaveRows) {
     const int me = base + lane;
@@ -1069,54 +1092,40 @@ __global__ __launch_bounds__(64) void k_sur_back_pairs(Buffers b, DevParams p, D
     }
     const PartInfo q = part_info(p, norm, raw);
     Cursor cu{0u, 0u, 0u, 0, me >= n, 0u, 0u, 0u, 0u, 0u, 0u, rr[0], rr[1], rr[2]};
-    for (;;) {
-      uint32_t t = 0;
-      float2 xj = make_float2(0.0f, 0.0f);
-      float Rx = 0.0f, Ry = 0.0f, r2 = 0.0f;
-      const bool have = next_pair(cu, p, src, q, me, false, t, xj, Rx, Ry, r2);
-      if (__ballot(have) == 0ull) break;  // wave-uniform
-      uint32_t w[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-      if (have) pair_words(w, src, p, norm, q, t, xj, Rx, Ry, r2);
+    auto masked = [&](const floatx16 &z, const floatx16 &d, int st) {
+      float v[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) fw[lane][k] = w[k];
-      const PairA a = pair_operands(w);
-      __syncthreads();
+      for (int u = 0; u < 8; ++u) v[u] = z[8 * st + u] > 0.0f ? d[8 * st + u] : 0.0f;
+      return pack_rows(v);
+    };
+    auto add_tile = [&](bf16x8 a, const floatx16 &dlo, const floatx16 &dhi) {
+      floatx16 zlo, zhi;
+      pair_layer(a, w1, zlo, zhi);
+      const floatx16 f = mfma16(a, unit, zero16());
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        floatx16 zlo, zhi;
-        pair_layer(t ? a.t1 : a.t0, w1, zlo, zhi);
-        const floatx16 &dlo = t ? d10 : d00;
-        const floatx16 &dhi = t ? d11 : d01;
-        // K step st: K index 8g + u is tile row c_row(8st + u, g), this lane's
-        // register 8st + u (A: masked dH of hidden c; B: that row's feature c)
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-          uint32_t bw[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            uint32_t hv[2];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-              const uint32_t wd = fw[32 * t + c_row(8 * st + 2 * q + e, g)][(c & 15) >> 1];
-              hv[e] = c < kFeat ? ((c & 1) ? (wd >> 16) : (wd & 0xffffu)) : 0u;
-            }
-            bw[q] = hv[0] | (hv[1] << 16);
-          }
-          float ml[8], mh[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            ml[u] = zlo[8 * st + u] > 0.0f ? dlo[8 * st + u] : 0.0f;
-            mh[u] = zhi[8 * st + u] > 0.0f ? dhi[8 * st + u] : 0.0f;
-          }
-          const bf16x8 bf = bf8(bw[0], bw[1], bw[2], bw[3]);
-          glo = mfma16(bf8(pack2(ml[0], ml[1]), pack2(ml[2], ml[3]), pack2(ml[4], ml[5]), pack2(ml[6], ml[7])), bf,
-                       glo);
-          ghi = mfma16(bf8(pack2(mh[0], mh[1]), pack2(mh[2], mh[3]), pack2(mh[4], mh[5]), pack2(mh[6], mh[7])), bf,
-                       ghi);
-        }
+      for (int st = 0; st < 2; ++st) {
+        const int r = 8 * st;
+        const bf16x8 bf = bf8(pack2(f[r], f[r + 1]), pack2(f[r + 2], f[r + 3]), pack2(f[r + 4], f[r + 5]),
+                              pack2(f[r + 6], f[r + 7]));
+        glo = mfma16(masked(zlo, dlo, st), bf, glo);
+        ghi = mfma16(masked(zhi, dhi, st), bf, ghi);
       }
-      __syncthreads();
-    }
+    };
+    auto walk = [&](const PairSrc &sp, auto rows) {
+      for (;;) {
+        uint32_t t = 0;
+        float2 xj = make_float2(0.0f, 0.0f);
+        float Rx = 0.0f, Ry = 0.0f, r2 = 0.0f;
+        const bool have = next_pair(cu, p, sp, q, me, rows(), t, xj, Rx, Ry, r2);
+        if (__ballot(have) == 0ull) break;  // wave-uniform
+        uint32_t w[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+        if (have) pair_words(w, sp, p, norm, q, t, xj, Rx, Ry, r2);
+        const PairA a = pair_operands(w);
+        add_tile(a.t0, d00, d01);
+        add_tile(a.t1, d10, d11);
+      }
+    };
+    pair_pass(src, pool, b, p, q, rr, me, n, cu, walk);
   }
   float *out = pairPart + (size_t)blockIdx.x * (kHid * kFeat);
   if (c < kFeat) {
