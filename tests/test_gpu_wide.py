@@ -90,3 +90,14 @@ def test_workgroups_across_scenes_and_past_the_binned_particles(cap):
             ref.add_particles(2, np.array([[0.3 * k, 0.2 * m]], np.float32))
     sim.close()
     ref.close()
+
+
+@pytest.mark.parametrize("box", [130.0, 512.0, 1480.0, 2078.0])
+def test_cell_starts_of_grids_of_many_scan_workgroups(box):
+    # 16,900 to 4.3 million cells: up to 4,217 scan workgroups, whose preceding totals are added eight in flight;
+    # particles in the first and last cells and in between
+    rng = np.random.RandomState(int(box))
+    pos = rng.uniform(-0.5 * box, 0.5 * box, (700, 2)).astype(np.float32)
+    pos[0], pos[1] = (-0.5 * box, -0.5 * box), (0.499 * box, 0.4995 * box)
+    pos[2:300] = (np.array([0.3 * box, 0.44 * box]) + rng.uniform(0, 3.0, (298, 2))).astype(np.float32)
+    _check(SceneSpec(box, box, 1.0, pos, planes=wall_planes(box, box)), SPHParams(), (0.0, -9.8), [1, 3])
