@@ -140,13 +140,13 @@ __device__ __forceinline__ bf16x8 selection(int s) {
   return bf8(w[0], w[1], w[2], w[3]);
 }
 
-// B operand (K = 16) of the 16 x 32 matrix with ones where k == n.
-__device__ __forceinline__ bf16x8 identity16() {
+// B operand (K = 16) of the 16 x 32 matrix with ones where k + first == n.
+__device__ __forceinline__ bf16x8 identity16(int first) {
   const int c = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
   uint32_t w[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int k = 8 * g + 2 * q;
+    const int k = first + 8 * g + 2 * q;
     w[q] = k == c ? 0x3F80u : (k + 1 == c ? 0x3F800000u : 0u);  // BF16 1.0
   }
   return bf8(w[0], w[1], w[2], w[3]);
@@ -154,12 +154,8 @@ __device__ __forceinline__ bf16x8 identity16() {
 
 constexpr int kWaveRows = 64;    // particles per wave in the pair kernels
 constexpr int kHbStride = 68;    // BF16 per row of the head operand buffer (padded)
-constexpr int kGStride = kHid + 1;
-constexpr int kHbBytes = kSurRows * kHbStride * 2;
-constexpr int kHeadBytes = kHbBytes + kSurRows * kGStride * 4;
 constexpr int kTileCap = 512;    // staged candidates (positions, previous positions, densities)
 constexpr int kStageBytes = 3 * kTileCap * 8;
-constexpr int kPoolBytes = kHeadBytes > kStageBytes ? kHeadBytes : kStageBytes;
 
 // Per-particle inputs of the pair layer.
 struct PartInfo {
@@ -521,23 +517,40 @@ __device__ __forceinline__ floatx16 by_row(const float *v) {
   return z;
 }
 
-// The head without LDS, for a forward that keeps no activations.  The pair sums
-// h[tile][hidden half] have the particle as their lane (column) and the hidden
-// units in their registers, so that a layer's packed outputs are, after one
-// exchange between the wave's halves, the next layer's operands, both row tiles
-// share the weights' operands, and lane l ends with all 64 values of G of
-// particle l for the output layer's FP32 sum (k ascending, as the training
-// forward adds them from LDS: the same products in the same order).  262,144
-// particles: one tile after the other through LDS 20 of the forward's 60 us,
-// all of it 46 us now.
-__device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_t np, const SurrogateBufs &m) {
+// The head, without LDS.  The pair sums h[tile][hidden half] have the particle
+// as their lane (column) and the hidden units in their registers, so that a
+// layer's packed outputs are, after one exchange between the wave's halves, the
+// next layer's operands, both row tiles share the weights' operands, and lane l
+// ends with all 64 values of G of particle l for the output layer's FP32 sum (k
+// ascending).  262,144 particles: one tile after the other through LDS 20 of
+// the forward's 60 us, all of it 46 us now.
+// TRAIN also writes the activations, whose layout has the hidden unit as the
+// lane: H and M, whose BF16 operands are the values kept, times the identity,
+// and G as a second product with the operands' roles exchanged.
+template <bool TRAIN>
+__device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_t np, const SurrogateBufs &m,
+                                              int base, int n) {
   const float *prm = m.params;
+  const int c = threadIdx.x & 31;
   const auto cnt = __builtin_amdgcn_permlane32_swap(__float_as_uint((float)np), __float_as_uint((float)np), false, false);
+  uint4 *act[2];
+  if (TRAIN)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) act[t] = m.act + (size_t)(2 * blockIdx.x + t) * kActWords;
+  auto store_operands = [&](const bf16x8 (&op)[2][4], int at) {
+    const bf16x8 e0 = identity16(0), e1 = identity16(16);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      if (base + 32 * t < n)  // the tile exists
+        store_tile_bf16(act[t] + at, mfma16(op[t][1], e1, mfma16(op[t][0], e0, zero16())),
+                        mfma16(op[t][3], e1, mfma16(op[t][2], e0, zero16())));
+  };
   bf16x8 op[2][4], om[2][4];  // H, M: tile, K step
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int y = 0; y < 2; ++y) k_operands(h[t][y], op[t][2 * y], op[t][2 * y + 1]);
+  if (TRAIN) store_operands(op, 0);
   // output half y of a layer for both tiles
   auto dense = [&](const uint16_t *W, int y, const bf16x8 (&in)[2][4], floatx16 &z0, floatx16 &z1) {
     z0 = zero16(), z1 = zero16();
@@ -561,7 +574,23 @@ __device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_
     }
     k_operands(z0, om[0][2 * y], om[0][2 * y + 1]);
     k_operands(z1, om[1][2 * y], om[1][2 * y + 1]);
-    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (TRAIN) {
+    store_operands(om, 4 * 64);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      if (base + 32 * t >= n) continue;
+      floatx16 lo = zero16(), hi = zero16();
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        lo = mfma16(om[t][s], load_wb16(m.w3b, kHid, 0, 16 * s), lo);
+        hi = mfma16(om[t][s], load_wb16(m.w3b, kHid, 32, 16 * s), hi);
+      }
+      const float b3lo = prm[kOffB3 + c], b3hi = prm[kOffB3 + 32 + c];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) lo[r] = relu(lo[r] + b3lo), hi[r] = relu(hi[r] + b3hi);
+      store_tile_f32(reinterpret_cast<float4 *>(act[t] + 8 * 64), (int)threadIdx.x, lo, hi);
+    }
   }
   // G = relu(W3 M + b3), FP32; then o = W4 G + b4
   float2 o = make_float2(prm[kOffB4], prm[kOffB4 + 1]);
@@ -584,7 +613,6 @@ __device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_
       o.x = __builtin_fmaf(prm[kOffW4 + 32 * y + k], v, o.x);
       o.y = __builtin_fmaf(prm[kOffW4 + kHid + 32 * y + k], v, o.y);
     }
-    __builtin_amdgcn_sched_barrier(0);
     asm volatile("" : "+v"(o.x), "+v"(o.y));  // a half of W4 in scalar registers at a time: both would spill
   }
   return o;
@@ -599,17 +627,11 @@ __device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_
 template <bool MULTI, bool TRAIN>
 __global__ __launch_bounds__(64, 2) void k_sur_forward(Buffers b, DevParams p, DevScene s0, int n, SurrogateBufs m,
                                                        int mode) {
-  // LDS: the staged candidates during the pair layer, then the head's operand
-  // rows (hb: H, then M, of one row tile as BF16) and G (FP32)
-  __shared__ __align__(16) unsigned char pool[kPoolBytes];
-  __shared__ float shCnt[kWaveRows];
-  uint16_t(*hb)[kHbStride] = reinterpret_cast<uint16_t(*)[kHbStride]>(pool);
-  float(*gbuf)[kGStride] = reinterpret_cast<float(*)[kGStride]>(pool + kHbBytes);
-  const int lane = threadIdx.x, c = lane & 31, g = lane >> 5;
+  __shared__ __align__(16) unsigned char pool[kStageBytes];
+  const int lane = threadIdx.x;
   const int base = (int)blockIdx.x * kWaveRows;
   const int me = base + lane;
-  const float *prm = m.params;
-  const float *norm = prm + kOffNorm;
+  const float *norm = m.params + kOffNorm;
   const W1Operands w1 = load_w1(m.w1b);
   const bf16x8 sel[2] = {selection(0), selection(1)};
   const PartRaw raw = part_raw(b, min(me, n - 1));  // a lane past n reads the last particle, unused
@@ -624,8 +646,7 @@ __global__ __launch_bounds__(64, 2) void k_sur_forward(Buffers b, DevParams p, D
   const PartInfo q = part_info(p, norm, raw);
   Cursor cu{0u, 0u, 0u, 0, me >= n, 0u, 0u, 0u, 0u, 0u, 0u, rr[0], rr[1], rr[2]};
   floatx16 h[2][2] = {{zero16(), zero16()}, {zero16(), zero16()}};  // tile, hidden half
-  // the training forward keeps the particle in the rows, the other in the lanes
-  auto add = [&](bf16x8 z, int s, floatx16 &acc) { acc = TRAIN ? mfma16(sel[s], z, acc) : mfma16(z, sel[s], acc); };
+  auto add = [&](bf16x8 z, int s, floatx16 &acc) { acc = mfma16(z, sel[s], acc); };
   auto add_tile = [&](bf16x8 a, floatx16 (&acc)[2]) {
     floatx16 zlo, zhi;
     pair_layer(a, w1, zlo, zhi);
@@ -653,111 +674,38 @@ __global__ __launch_bounds__(64, 2) void k_sur_forward(Buffers b, DevParams p, D
     }
   };
   pair_pass(src, pool, b, p, q, rr, me, n, cu, walk);
-  auto pair_total = [&] {
-    if (!m.pairPart) return;
+
+  // 2. head
+  if (TRAIN && me < n) m.cnt[me] = (float)np;
+  const float2 o = head_output<TRAIN>(h, np, m, base, n);
+  if (m.pairPart) {
     uint32_t tot = np;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) tot += (uint32_t)__shfl_xor((int)tot, off, 64);
     if (lane == 0) m.pairPart[blockIdx.x] = tot;
-  };
-  // o of particle i: the network's output, and the state after the relaxation
-  // and the boundary collisions
-  auto finish = [&](int i, bool live, float2 o) {
-    if (live && m.out) reinterpret_cast<float2 *>(m.out)[i] = o;
-    if (!(mode & kFwdState)) return;
-    DevScene sc = s0;
-    float x = 0.0f, y = 0.0f;
-    if (live) {
-      sc = scene_of_slot<MULTI>(b, s0, b.keys[i]);
-      const float2 xi = b.x1[i];
-      x = xi.x + o.x * norm[5];
-      y = xi.y + o.y * norm[5];
-    }
-    collide_wave<MULTI>(b, p, sc, x, y, live);                                 // demo4.cpp:411-444
-    if (live) {
-      if (mode & kFwdPressure) {
-        const float2 d = b.dens[i];
-        b.pres[i] = make_float2(p.k * (d.x - p.rho0), p.kn * d.y);             // sph.h:478-481
-      }
-      const float2 pv = b.prev[i];
-      b.x0[i] = make_float2(x, y);
-      b.v[i] = make_float2((x - pv.x) * p.invDt, (y - pv.y) * p.invDt);        // demo4.cpp:446-450
-    }
-  };
-  if constexpr (!TRAIN) {
-    const float2 o = head_output(h, np, m);
-    pair_total();
-    finish(me, me < n, o);
-    return;
   }
-  // (TRAIN from here on)
-  pair_total();
-  shCnt[lane] = (float)np;
-
-  // 2. head, one 32-row tile at a time: C = A W^T with A in hb (BF16)
-  auto dense = [&](const uint16_t *W, floatx16 &olo, floatx16 &ohi) {
-    bf16x8 a[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) a[s] = lds_bf8(&hb[c][16 * s + 8 * g]);
-    olo = zero16();
-    ohi = zero16();
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      olo = mfma16(a[s], load_wb16(W, kHid, 0, 16 * s), olo);
-      ohi = mfma16(a[s], load_wb16(W, kHid, 32, 16 * s), ohi);
+  // 3. the network's output, and the state after the relaxation and the
+  // boundary collisions
+  const bool live = me < n;
+  if (live && m.out) reinterpret_cast<float2 *>(m.out)[me] = o;
+  if (!(mode & kFwdState)) return;
+  DevScene sc = s0;
+  float x = 0.0f, y = 0.0f;
+  if (live) {
+    sc = scene_of_slot<MULTI>(b, s0, b.keys[me]);
+    const float2 xi = b.x1[me];
+    x = xi.x + o.x * norm[5];
+    y = xi.y + o.y * norm[5];
+  }
+  collide_wave<MULTI>(b, p, sc, x, y, live);                                   // demo4.cpp:411-444
+  if (live) {
+    if (mode & kFwdPressure) {
+      const float2 d = b.dens[me];
+      b.pres[me] = make_float2(p.k * (d.x - p.rho0), p.kn * d.y);              // sph.h:478-481
     }
-  };
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const floatx16 &hlo = h[t][0];
-    const floatx16 &hhi = h[t][1];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int row = c_row(k, g);
-      hb[row][c] = f2bf(hlo[k]);
-      hb[row][32 + c] = f2bf(hhi[k]);
-    }
-    __syncthreads();
-    const int i = base + 32 * t + c;  // A-operand row c of this tile
-    uint4 *const act = TRAIN ? m.act + (size_t)(2 * blockIdx.x + t) * kActWords : nullptr;
-    const bool rowsLive = base + 32 * t < n;  // the tile exists
-    if (TRAIN && rowsLive) {
-      store_tile_bf16(act, hlo, hhi);
-      if (g == 0 && i < n) m.cnt[i] = shCnt[32 * t + c];
-    }
-    // M = W2 H + n b2, kept as BF16 in hb
-    floatx16 olo, ohi;
-    dense(m.w2b, olo, ohi);
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int row = c_row(k, g);
-      const float nc = shCnt[32 * t + row];
-      olo[k] += nc * prm[kOffB2 + c];
-      ohi[k] += nc * prm[kOffB2 + 32 + c];
-      hb[row][c] = f2bf(olo[k]);
-      hb[row][32 + c] = f2bf(ohi[k]);
-    }
-    __syncthreads();
-    if (TRAIN && rowsLive) store_tile_bf16(act + 4 * 64, olo, ohi);
-    // G = relu(W3 M + b3), FP32
-    dense(m.w3b, olo, ohi);
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int row = c_row(k, g);
-      olo[k] = relu(olo[k] + prm[kOffB3 + c]);
-      ohi[k] = relu(ohi[k] + prm[kOffB3 + 32 + c]);
-      gbuf[row][c] = olo[k];
-      gbuf[row][32 + c] = ohi[k];
-    }
-    __syncthreads();
-    if (TRAIN && rowsLive) store_tile_f32(reinterpret_cast<float4 *>(act + 8 * 64), lane, olo, ohi);
-    // 3. o = W4 G + b4 (FP32): lane (c, g) computes output g of particle i
-    float o = prm[kOffB4 + g];
-    for (int k = 0; k < kHid; ++k) o = __builtin_fmaf(prm[kOffW4 + g * kHid + k], gbuf[c][k], o);
-    const float oy = __shfl_down(o, 32, 64);
-    finish(i, g == 0 && i < n, make_float2(o, oy));
+    const float2 pv = b.prev[me];
+    b.x0[me] = make_float2(x, y);
+    b.v[me] = make_float2((x - pv.x) * p.invDt, (y - pv.y) * p.invDt);         // demo4.cpp:446-450
   }
 }
 
@@ -1067,7 +1015,7 @@ __global__ __launch_bounds__(64, 2) void k_sur_back_pairs(Buffers b, DevParams p
   const int lane = threadIdx.x, c = lane & 31, g = lane >> 5;
   const float *norm = m.params + kOffNorm;
   const W1Operands w1 = load_w1(m.w1b);
-  const bf16x8 unit = identity16();
+  const bf16x8 unit = identity16(0);
   floatx16 glo = zero16(), ghi = zero16();
   for (int base = (int)blockIdx.x * kWaveRows; base < n; base += (int)gridDim.x * kWaveRows) {
     const int me = base + lane;
