@@ -519,9 +519,10 @@ __device__ __forceinline__ void open_block(const Buffers &b, const DevScene &s0,
 // formed in 32 bits (the difference wraps).  Entries past the end are clamped
 // to the last one, which is then loaded and stored more than once with the
 // same value.
-template <int N>
-__device__ __forceinline__ void stage_arrays(const TilePlan &t, const float2 *const (&src)[N],
-                                             float2 *const (&dst)[N]) {
+// map(v) turns an entry's N values into the ones stored.
+template <int N, typename Map>
+__device__ __forceinline__ void stage_arrays(const TilePlan &t, const float2 *const (&src)[N], float2 *const (&dst)[N],
+                                             Map &&map) {
   constexpr uint32_t kU = 4;
   const uint32_t total = t.off[3], off1 = t.off[1], off2 = t.off[2];
   const uint32_t b0 = t.rowStart[0] - t.off[0], b1 = t.rowStart[1] - off1, b2 = t.rowStart[2] - off2;
@@ -536,16 +537,21 @@ __device__ __forceinline__ void stage_arrays(const TilePlan &t, const float2 *co
       for (int a = 0; a < N; ++a) v[a][u] = src[a][(uint32_t)(at[u] + b)];
     }
 #pragma unroll
-    for (uint32_t u = 0; u < kU; ++u)
+    for (uint32_t u = 0; u < kU; ++u) {
+      float2 w[N];
 #pragma unroll
-      for (int a = 0; a < N; ++a) dst[a][at[u]] = v[a][u];
+      for (int a = 0; a < N; ++a) w[a] = v[a][u];
+      map(w);
+#pragma unroll
+      for (int a = 0; a < N; ++a) dst[a][at[u]] = w[a];
+    }
   }
 }
 
 __device__ __forceinline__ void stage(const TilePlan &t, const float2 *src, float2 *dst) {
   const float2 *const s[1] = {src};
   float2 *const d[1] = {dst};
-  stage_arrays<1>(t, s, d);
+  stage_arrays<1>(t, s, d, [](float2 (&)[1]) {});
 }
 
 // A float held in a vector register: an FP32 instruction with a scalar operand
@@ -556,6 +562,27 @@ __device__ __forceinline__ float in_vgpr(float s) {
   asm("v_mov_b32 %0, %1" : "=v"(v) : "s"(s));
   return v;
 }
+
+// Whether near_length serves this wave's active lanes: h > 2^-36, and no
+// particle with |x| or |y| below 2^-23 (two different floats of which one is
+// 2^-23 or more differ by 2^-47 or more, so every pair of such a particle has
+// r2 == 0 or r2 >= 2^-96).
+__device__ __forceinline__ bool wave_near(const DevParams &p, float2 x) {
+  return p.h > 0x1p-36f && __ballot(fminf(fabsf(x.x), fabsf(x.y)) < 0x1p-23f) == 0ull;
+}
+// The pair length by near_length or pair_length; near is wave-uniform, and a
+// compile-time constant in the one-lane-per-particle walks, whose four slots
+// then share one block without branches.  pair_length's branch for tiny r2 was
+// taken by nearly every wave there, since r2 == 0 for a particle and itself:
+// 1,048,576 particles (step 480) viscosity 91 -> 76 us, density 61 -> 54, delta
+// 91 -> 77.
+__device__ __forceinline__ void length_of(bool near, float r2, float &r, float &inv) {
+  if (near)
+    near_length(r2, r, inv);
+  else
+    pair_length(r2, r, inv);
+}
+__device__ __forceinline__ float root_of(bool near, float r2) { return near ? near_sqrt(r2) : pair_sqrt(r2); }
 
 // Index of slot j of row range d in the neighbour data source.
 struct TileIndex {

@@ -30,27 +30,6 @@
 
 namespace nbs {
 
-// Whether near_length serves this wave's active lanes: h > 2^-36, and no
-// particle with |x| or |y| below 2^-23 (two different floats of which one is
-// 2^-23 or more differ by 2^-47 or more, so every pair of such a particle has
-// r2 == 0 or r2 >= 2^-96).
-__device__ __forceinline__ bool wave_near(const DevParams &p, float2 x) {
-  return p.h > 0x1p-36f && __ballot(fminf(fabsf(x.x), fabsf(x.y)) < 0x1p-23f) == 0ull;
-}
-// The pair length by near_length or pair_length; near is wave-uniform, and a
-// compile-time constant in the one-lane-per-particle walks, whose four slots
-// then share one block without branches.  pair_length's branch for tiny r2 was
-// taken by nearly every wave there, since r2 == 0 for a particle and itself:
-// 1,048,576 particles (step 480) viscosity 91 -> 76 us, density 61 -> 54, delta
-// 91 -> 77.
-__device__ __forceinline__ void length_of(bool near, float r2, float &r, float &inv) {
-  if (near)
-    near_length(r2, r, inv);
-  else
-    pair_length(r2, r, inv);
-}
-__device__ __forceinline__ float root_of(bool near, float r2) { return near ? near_sqrt(r2) : pair_sqrt(r2); }
-
 // For every candidate slot j (of the three row ranges) of the particle at xi whose
 // r2 < h2 (sph.h:470, 488, 502), in candidate order, applies the pair's
 // contribution: apply(term(j, Rx, Ry, r2, true)).  term(..., false) must return
