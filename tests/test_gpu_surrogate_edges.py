@@ -47,3 +47,18 @@ def test_inference_and_training_forward_agree(sizes, spacing):
             states.append(sim.get_state())
     for k in ("x", "v", "density"):
         assert np.array_equal(states[0][k].view(np.uint32), states[1][k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("n,spacing", [(65, 0.12), (300, 0.12), (700, 0.06)])
+def test_gradient_of_crowded_rows(n, spacing):
+    # rows of more than 32 candidates, up to three chunks of them buffered per lane, some lanes without pairs
+    cols = int(np.ceil(np.sqrt(n)))
+    pos = volume_positions((0.0, 0.0), cols, cols, spacing, 1.0, seed=n, limit=n)
+    pos[-5:] += np.array([[4.0, 4.0]], np.float32) * np.arange(1, 6, dtype=np.float32)[:, None] / 2
+    with ParticleSimulation.from_scene(SceneSpec(32.0, 32.0, 1.0, pos, planes=wall_planes(32.0, 32.0)),
+                                       SPHParams(k=1e-4, k_near=1e-4), GRAVITY) as sim:
+        rng = np.random.RandomState(n)
+        sim.set_state(pos, rng.normal(0.0, 0.1, pos.shape).astype(np.float32))
+        sim.surrogate_init(3)
+        sim.surrogate_calibrate(DT)
+        check_frame(sim)
