@@ -1140,14 +1140,19 @@ __global__ __launch_bounds__(kBlock) void k_visc_predict_wide(Buffers b, DevPara
     pcx = (int)local - pcy * sc.nx;
     float accx = 0.0f, accy = 0.0f;
     const bool near = wave_near(p, xi);
+    // u > 0 (below) needs s = (v_i - v_j) . R > 0 up to rounding, so pairs that
+    // separate are not listed (half of them).  With R's components 0 or at least
+    // 2^-47 and r < 2^20, n's are normal, and u is s / r up to 2^-22 of its two
+    // products and 2^-149: an s below -2^-16 of its own products and below
+    // -2^-126 (so that their underflow counts for nothing, and |s| / r is at
+    // least 2^-146) has u <= 0.  In other waves every pair is listed.
+    const float margin = near && p.h <= 0x1p20f ? 0x1p-126f : __builtin_inff();
     for_each_pair_wide<G, true>(
         b.startCur, sc, pcx, pcy, b.x0, b.v, (uint32_t)i, xi, p.h2, list + group * (kGroupList * G),
         [&](float Rx, float Ry, float, float2 vj, float4 &e) {
           e = make_float4(Rx, Ry, p.gdtx + vj.x, p.gdty + vj.y);
-          // u > 0 (below) needs (v_i - v_j) . R > 0 up to rounding: pairs that
-          // separate are not listed (half of them)
           const float a = (vx - e.z) * Rx, c = (vy - e.w) * Ry;
-          return !(a + c < -0x1p-16f * (fabsf(a) + fabsf(c)));
+          return !(a + c < -0x1p-16f * (fabsf(a) + fabsf(c)) - margin);
         },
         [&](float4 e, bool in, int left) {
           const float r2 = e.x * e.x + e.y * e.y;
