@@ -166,6 +166,14 @@ __device__ __forceinline__ void group_apply(int left, F &&f) {
   }
 }
 
+// Orders the wave's LDS accesses before and after it, for lanes that read what
+// others wrote.  The hardware runs one wave's LDS operations in order, so this
+// only keeps the compiler from moving them and issues nothing.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <int G, bool VALUES, typename Entry, typename Keep, typename Use>
 __device__ __forceinline__ uint32_t for_each_pair_wide(const uint32_t *start, const DevScene &sc, int cx, int cy,
                                                        const float2 *X, const float2 *V, uint32_t own, float2 xi,
@@ -180,15 +188,18 @@ __device__ __forceinline__ uint32_t for_each_pair_wide(const uint32_t *start, co
   const uint32_t b0 = rr[0].j0 + sub, b1 = rr[1].j0 - c0 * G + sub, b2 = rr[2].j0 - c1 * G + sub;
   uint32_t cnt = 0;
   if (sub == 0u) list[0] = Entry{};  // read by the lanes past a group's end, also when it never has a pair
+  wave_lds_order();                  // before another lane's first entry
   for (uint32_t k0 = 0;; k0 += kAhead) {
     const bool done = __ballot(k0 < chunks) == 0ull;  // wave-uniform
     if (done || __ballot(cnt > kCap - kAhead * G)) {
+      wave_lds_order();  // the lanes' entries, before the group reads them
       for (uint32_t q = 0; __ballot(q < cnt); q += G) {
         const bool in = q + sub < cnt;
         // the entries past the middle of the batch: applied only when some group has them
         const bool half = G == 16 && __ballot(q + 8u < cnt) == 0ull;
         use(list[in ? q + sub : 0u], in, half ? G / 2 : G);
       }
+      wave_lds_order();  // the entries have been read
       cnt = 0u;
       if (done) break;
     }
