@@ -119,6 +119,8 @@ class PinnedBuffer {
     }
     (void)hipHostFree(p_);
   }
+  // The buffer, or null when the system refuses pinned memory (its limit is not
+  // the device's); the callers then copy straight to pageable memory.
   uint8_t *get() {
     if (p_) return p_;
     {
@@ -130,8 +132,10 @@ class PinnedBuffer {
       }
     }
     void *p = nullptr;
-    const hipError_t e = hipHostMalloc(&p, kPinnedBytes, hipHostMallocPortable);
-    if (e != hipSuccess) throw Error(NBS_ERR_OUT_OF_MEMORY, std::string("hipHostMalloc: ") + hipGetErrorString(e));
+    if (hipHostMalloc(&p, kPinnedBytes, hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();  // or the next launch would report it
+      return nullptr;
+    }
     return p_ = static_cast<uint8_t *>(p);
   }
 
@@ -338,8 +342,8 @@ class Simulation {
       NBS_HIP(hipGetLastError());
     }
     const size_t bytes = 8 * n_;
-    if (2 * bytes <= kPinnedBytes) {
-      uint8_t *pin = pinned_.get();
+    uint8_t *const pin = 2 * bytes <= kPinnedBytes ? pinned_.get() : nullptr;
+    if (pin) {
       std::memcpy(pin, x, bytes);
       std::memcpy(pin + bytes, v, bytes);
       NBS_HIP(hipMemcpyAsync(st.x, pin, 2 * bytes, hipMemcpyHostToDevice, stream_));  // st.x, st.prev
@@ -777,14 +781,15 @@ class Simulation {
     size_t bytes;
   };
   // Copies the wanted arrays to the host and waits for them: through pinned
-  // memory when they are small together, else straight; one copy per run of
-  // arrays that are adjacent (on both sides for the straight ones).
+  // memory when they are small together (and there is pinned memory), else
+  // straight; one copy per run of arrays that are adjacent (on both sides for
+  // the straight ones).
   void readBack(const Readback *all, int count) {
     size_t total = 0;
     for (int k = 0; k < count; ++k)
       if (all[k].dst) total += all[k].bytes;
-    const bool pin = total <= kPinnedBytes;
-    uint8_t *const stage = pin && total ? pinned_.get() : nullptr;
+    uint8_t *const stage = total && total <= kPinnedBytes ? pinned_.get() : nullptr;
+    const bool pin = stage != nullptr;
     size_t at = 0;
     for (int k = 0; k < count;) {
       size_t bytes = all[k].bytes;
