@@ -206,9 +206,11 @@ nbs_status nbs_set_options(nbs_sim *sim, uint32_t flags);
  * workgroup's candidate rows in LDS tiles of tile_cap particles (0: no staging,
  * read neighbours from HBM/L2).  With autotune on, the library times every capacity on real steps
  * (all capacities give bit-identical results) and keeps the fastest per
- * kernel, again every retune_interval steps (0: once; default 256); steps of
- * at most 65,536 particles use the wide kernels.  No reference
- * counterpart: the reference's only tunable is its thread count. */
+ * kernel, again every retune_interval steps (0: once; default 256).  Steps of
+ * at most 65,536 particles use the wide kernels instead, and nbs_get_tuning
+ * then reports -1 for them; an earlier tuning's capacities (autotune = 2) are
+ * used from 1,024 particles on.  No reference counterpart: the reference's only
+ * tunable is its thread count. */
 typedef struct nbs_tuning {
   int32_t autotune;          /* 0: tile_cap fixed; 1: tune now, then every retune_interval steps;
                                 2: as 1, with tile_cap taken as an earlier tuning's result (no first tuning;

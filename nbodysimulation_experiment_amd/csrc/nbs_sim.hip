@@ -503,12 +503,18 @@ class Simulation {
     // re-tuning runs.
     tuned_ = t.autotune == 2;
     if (tuning_.autotune == 2) tuning_.autotune = 1;
+    savedCaps_ = tuned_ && std::any_of(t.tile_cap, t.tile_cap + 3, [](int32_t c) { return c != kWideCap; });
+    ranWide_ = false;
     tuneActive_ = false;
     tunePending_.clear();
     stepsSinceTune_ = 0;
     destroyGraph();
   }
-  nbs_tuning tuning() const { return tuning_; }
+  nbs_tuning tuning() const {
+    nbs_tuning t = tuning_;
+    if (ranWide_ && wideByRule()) std::fill(t.tile_cap, t.tile_cap + 3, kWideCap);
+    return t;
+  }
 
   hipStream_t stream() const { return stream_; }
 
@@ -980,9 +986,12 @@ class Simulation {
   // tile capacity, or kWideCap for small steps.
   // Wide kernels for every phase: below the autotuner's range, where they are
   // the fastest for every packing, or up to nbs_tuning.wide_max_particles.
+  // Capacities that the caller brought as an earlier tuning's result are used
+  // (and retuned) from 1,024 particles on, where such tunings were made.
+  static constexpr uint64_t kSavedCapsMin = 1024;
+  bool wideByRule() const { return tuning_.autotune && n_ <= (savedCaps_ ? kSavedCapsMin - 1 : kWideParticles); }
   bool wideStep() const {
-    return (tuning_.autotune && n_ <= kWideParticles) ||
-           (tuning_.wide_max_particles > 0 && n_ <= (uint64_t)tuning_.wide_max_particles);
+    return wideByRule() || (tuning_.wide_max_particles > 0 && n_ <= (uint64_t)tuning_.wide_max_particles);
   }
   void pairCaps(int cap[3]) const {
     for (int k = 0; k < 3; ++k) cap[k] = wideStep() ? kWideCap : tuning_.tile_cap[k];
@@ -999,6 +1008,7 @@ class Simulation {
     const int n = (int)n_;
     int cap[3];
     pairCaps(cap);
+    ranWide_ = ranWide_ || wideByRule();
     // Placement binning: the viscosity kernel lists the far movers, k_place
     // orders and moves; on large grids every step's scan clears the counter
     // of the next step's parity.
@@ -1541,6 +1551,8 @@ class Simulation {
   std::vector<std::pair<uint32_t, uint32_t>> tunePending_;  // (event slot, candidate) of this call
   uint64_t stepsSinceTune_ = 0;
   uint64_t tuneCount_ = 0;
+  bool savedCaps_ = false;  // tile_cap came from the caller as an earlier tuning's result, not all wide
+  bool ranWide_ = false;    // a step since the tuning was set took the wide kernels by rule
 
   hipGraphExec_t graphExec_ = nullptr;
   DevParams graphParams_{};

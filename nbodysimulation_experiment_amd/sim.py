@@ -308,8 +308,10 @@ class ParticleSimulation:
                    wide_max_particles: int = 0, tuned: bool = False):
         """autotune: time the kernel variants on real steps (first all of them,
         then every retune_interval steps the current choice and its
-        neighbours); tuned=True takes tile_cap as an earlier tuning's result,
-        so only the periodic re-tuning runs."""
+        neighbours), or the wide kernels for at most 65,536 particles, which
+        get_tuning then reports as -1; tuned=True takes tile_cap as an earlier
+        tuning's result, used from 1,024 particles on, so only the periodic
+        re-tuning runs."""
         mode = (2 if tuned else 1) if autotune else 0
         t = NbsTuning(mode, int(retune_interval), (ctypes.c_int32 * 3)(*tile_cap), int(wide_max_particles))
         call("nbs_set_tuning", self._h, ctypes.byref(t))
