@@ -1020,6 +1020,24 @@ __global__ __launch_bounds__(kUpdateBlock) void k_grad_update(const float *pairP
   }
 }
 
+// B operand (16 rows x 32 features, 16 used) of K step st of the row tile from
+// row0: K index 8g + u is row c_row(8 st + u, g).
+__device__ __forceinline__ bf16x8 lds_features(const uint32_t (*fw)[kFeat / 2], int row0, int st) {
+  const int c = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
+  uint32_t w[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    uint32_t v[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const uint32_t word = fw[row0 + c_row(8 * st + 2 * q + e, g)][(c & 15) >> 1];
+      v[e] = c < kFeat ? ((c & 1) ? word >> 16 : word & 0xffffu) : 0u;
+    }
+    w[q] = v[0] | (v[1] << 16);
+  }
+  return bf8(w[0], w[1], w[2], w[3]);
+}
+
 // dW1 = sum_i sum_j (dH_i . [z_ij > 0]) f_ij^T, with the pair walk of the
 // forward pass.  For row tile t the pair layer's pre-activations (C layout:
 // lane = hidden unit, register r = tile row c_row(r, g)), masked and scaled by
@@ -1030,15 +1048,23 @@ __global__ __launch_bounds__(kUpdateBlock) void k_grad_update(const float *pairP
 // words read per tile and lane and taken apart, a 327,680-particle launch took
 // 135 us instead of 63).  Each wave accumulates over its particles and writes
 // one 64 x 16 partial.
+// The product passes a row on only if all its features are finite: a NaN or an
+// infinity times the identity's zeros makes the whole row NaN.  The 16 unused
+// columns, zero otherwise, show it in the sums, and such a wave starts again
+// with the features through LDS, each of which reaches its own column alone.
 template <bool MULTI>
 __global__ __launch_bounds__(64, 2) void k_sur_back_pairs(Buffers b, DevParams p, DevScene s0, int n, SurrogateBufs m,
                                                           float *pairPart) {
   __shared__ __align__(16) unsigned char pool[kStageBytes];
+  __shared__ uint32_t fw[kWaveRows][kFeat / 2];  // the pairs' features, when they are not finite
   const int lane = threadIdx.x, c = lane & 31, g = lane >> 5;
   const float *norm = m.params + kOffNorm;
   const W1Operands w1 = load_w1(m.w1b);
   const bf16x8 unit = identity16(0);
-  floatx16 glo = zero16(), ghi = zero16();
+  floatx16 glo, ghi;
+  bool exact = false;  // wave-uniform
+again:
+  glo = zero16(), ghi = zero16();
   for (int base = (int)blockIdx.x * kWaveRows; base < n; base += (int)gridDim.x * kWaveRows) {
     const int me = base + lane;
     __syncthreads();  // the previous group's tile is no longer read
@@ -1069,20 +1095,21 @@ __global__ __launch_bounds__(64, 2) void k_sur_back_pairs(Buffers b, DevParams p
       for (int u = 0; u < 8; ++u) v[u] = z[8 * st + u] > 0.0f ? d[8 * st + u] : 0.0f;
       return pack_rows(v);
     };
-    auto add_tile = [&](bf16x8 a, const floatx16 &dlo, const floatx16 &dhi) {
+    auto add_tile = [&](int t, bf16x8 a, const floatx16 &dlo, const floatx16 &dhi, auto viaLds) {
       floatx16 zlo, zhi;
       pair_layer(a, w1, zlo, zhi);
       const floatx16 f = mfma16(a, unit, zero16());
 #pragma unroll
       for (int st = 0; st < 2; ++st) {
         const int r = 8 * st;
-        const bf16x8 bf = bf8(pack2(f[r], f[r + 1]), pack2(f[r + 2], f[r + 3]), pack2(f[r + 4], f[r + 5]),
-                              pack2(f[r + 6], f[r + 7]));
+        const bf16x8 bf = viaLds() ? lds_features(fw, 32 * t, st)
+                                   : bf8(pack2(f[r], f[r + 1]), pack2(f[r + 2], f[r + 3]), pack2(f[r + 4], f[r + 5]),
+                                         pack2(f[r + 6], f[r + 7]));
         glo = mfma16(masked(zlo, dlo, st), bf, glo);
         ghi = mfma16(masked(zhi, dhi, st), bf, ghi);
       }
     };
-    auto walk = [&](const PairSrc &sp, auto rows) {
+    auto pairs = [&](const PairSrc &sp, auto rows, auto viaLds) {
       for (;;) {
         uint32_t t = 0;
         float2 xj = make_float2(0.0f, 0.0f);
@@ -1091,12 +1118,31 @@ __global__ __launch_bounds__(64, 2) void k_sur_back_pairs(Buffers b, DevParams p
         if (__ballot(have) == 0ull) break;  // wave-uniform
         uint32_t w[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
         if (have) pair_words(w, sp, p, norm, q, t, xj, Rx, Ry, r2, near);
+        if (viaLds()) {
+          __syncthreads();  // the last iteration's features have been read
+#pragma unroll
+          for (int k = 0; k < kFeat / 2; ++k) fw[lane][k] = w[k];
+          __syncthreads();
+        }
         const PairA a = pair_operands(w);
-        add_tile(a.t0, d00, d01);
-        add_tile(a.t1, d10, d11);
+        add_tile(0, a.t0, d00, d01, viaLds);
+        add_tile(1, a.t1, d10, d11, viaLds);
       }
     };
-    pair_pass(src, pool, b, p, q, rr, me, n, cu, walk);
+    if (exact)  // one copy of the walk for all
+      pairs(slot_src(src, b), std::false_type(), std::true_type());
+    else
+      pair_pass(src, pool, b, p, q, rr, me, n, cu,
+                [&](const PairSrc &sp, auto rows) { pairs(sp, rows, std::false_type()); });
+  }
+  if (!exact) {
+    float unused = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) unused += glo[k] + ghi[k];
+    if (__ballot(c >= kFeat && unused != 0.0f) != 0ull) {  // NaN
+      exact = true;
+      goto again;
+    }
   }
   float *out = pairPart + (size_t)blockIdx.x * (kHid * kFeat);
   if (c < kFeat) {
