@@ -115,6 +115,13 @@ __device__ __forceinline__ bf16x8 lds_bf8(const uint16_t *p) {
   return bf8(w[0], w[1], w[2], w[3]);
 }
 
+__device__ __forceinline__ void lds_put8(uint16_t *p, bf16x8 v) {
+  const u32x4 u = __builtin_bit_cast(u32x4, v);
+  uint32_t *w = reinterpret_cast<uint32_t *>(p);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) w[k] = u[k];
+}
+
 // B operand of step s (K = 16 rows of a 32-row C-layout tile z): this lane's
 // registers 8s .. 8s + 7, relu'd in BF16.
 __device__ __forceinline__ bf16x8 relu_rows(const floatx16 &z, int s) {
@@ -156,6 +163,7 @@ constexpr int kWaveRows = 64;    // particles per wave in the pair kernels
 constexpr int kHbStride = 68;    // BF16 per row of the head operand buffer (padded)
 constexpr int kTileCap = 512;    // staged candidates (positions, previous positions, densities)
 constexpr int kStageBytes = 3 * kTileCap * 8;
+static_assert(kSurRows * kHbStride * 2 <= kStageBytes, "a row tile's BF16 activations fit the staging pool");
 
 // Per-particle inputs of the pair layer.
 struct PartInfo {
@@ -509,6 +517,12 @@ __device__ __forceinline__ void store_tile_bf16(uint4 *dst, floatx16 lo, floatx1
   dst[2 * 64 + threadIdx.x] = pack8(hi, 0);
   dst[3 * 64 + threadIdx.x] = pack8(hi, 1);
 }
+// One word of it from LDS: particles 16 s + 8 g + {0 .. 7} of hidden column h.
+__device__ __forceinline__ uint4 lds_column(const uint16_t (*rows)[kHbStride], int h, int s) {
+  const uint16_t(*r)[kHbStride] = rows + 16 * s + 8 * (int)((threadIdx.x >> 5) & 1);
+  auto two = [&](int k) { return (uint32_t)r[k][h] | ((uint32_t)r[k + 1][h] << 16); };
+  return make_uint4(two(0), two(2), two(4), two(6));
+}
 // Word q of an FP32 tile: rows 2q and 2q + 1 of the lane's two columns.
 __device__ __forceinline__ void store_tile_f32(float4 *dst, int lane, const floatx16 &lo, const floatx16 &hi) {
 #pragma unroll
@@ -547,10 +561,14 @@ __device__ __forceinline__ floatx16 by_row(const float *v) {
 // the forward's 60 us, all of it 46 us after.
 // TRAIN also writes the activations, whose layout has the hidden unit as the
 // lane: H and M, whose BF16 operands are the values kept, times the identity,
-// and G as a second product with the operands' roles exchanged.
+// and G as a second product with the operands' roles exchanged.  An infinite or
+// NaN value times the identity's zeros would make its particle's others NaN, so
+// a wave that holds one stores them again, transposed through LDS (pool); it
+// shows in any one of the next layer's pre-activations, which add infinity or
+// NaN times a weight.
 template <bool TRAIN>
 __device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_t np, const SurrogateBufs &m,
-                                              int base, int n) {
+                                              int base, int n, unsigned char *pool) {
   const float *prm = m.params;
   const int c = threadIdx.x & 31;
   const auto cnt = __builtin_amdgcn_permlane32_swap(__float_as_uint((float)np), __float_as_uint((float)np), false, false);
@@ -566,6 +584,20 @@ __device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_
         store_tile_bf16(act[t] + at, mfma16(op[t][1], e1, mfma16(op[t][0], e0, zero16())),
                         mfma16(op[t][3], e1, mfma16(op[t][2], e0, zero16())));
   };
+  auto store_through_lds = [&](const bf16x8 (&op)[2][4], int at) {
+    uint16_t(*rows)[kHbStride] = reinterpret_cast<uint16_t(*)[kHbStride]>(pool);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      __syncthreads();  // pool is no longer read
+#pragma unroll
+      for (int s = 0; s < 4; ++s) lds_put8(&rows[c][16 * s + 8 * (int)(threadIdx.x >> 5)], op[t][s]);
+      __syncthreads();
+      if (base + 32 * t >= n) continue;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) act[t][at + k * 64 + threadIdx.x] = lds_column(rows, 32 * (k >> 1) + c, k & 1);
+    }
+  };
+  bool finite = true;
   bf16x8 op[2][4], om[2][4];  // H, M: tile, K step
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -587,6 +619,7 @@ __device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_
   for (int y = 0; y < 2; ++y) {
     floatx16 z0, z1;
     dense(m.w2b, y, op, z0, z1);
+    if (y == 0) finite = finite && __builtin_isfinite(z0[0]) && __builtin_isfinite(z1[0]);
     const floatx16 b2 = by_row(prm + kOffB2 + 32 * y);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -619,6 +652,7 @@ __device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_
   for (int y = 0; y < 2; ++y) {
     floatx16 z0, z1;
     dense(m.w3b, y, om, z0, z1);
+    if (y == 0) finite = finite && __builtin_isfinite(z0[0]) && __builtin_isfinite(z1[0]);
     const floatx16 b3 = by_row(prm + kOffB3 + 32 * y);
     floatx16 g[2];  // rows c_row(r, 0), c_row(r, 1) of the lane's own particle
 #pragma unroll
@@ -635,6 +669,10 @@ __device__ __forceinline__ float2 head_output(const floatx16 (&h)[2][2], uint32_
       o.y = __builtin_fmaf(prm[kOffW4 + kHid + 32 * y + k], v, o.y);
     }
     asm volatile("" : "+v"(o.x), "+v"(o.y));  // a half of W4 in scalar registers at a time: both would spill
+  }
+  if (TRAIN && __ballot(!finite) != 0ull) {  // again, over the first stores
+    store_through_lds(op, 0);
+    store_through_lds(om, 4 * 64);
   }
   return o;
 }
@@ -699,7 +737,7 @@ __global__ __launch_bounds__(64, 2) void k_sur_forward(Buffers b, DevParams p, D
 
   // 2. head
   if (TRAIN && me < n) m.cnt[me] = (float)np;
-  const float2 o = head_output<TRAIN>(h, np, m, base, n);
+  const float2 o = head_output<TRAIN>(h, np, m, base, n, pool);
   if (m.pairPart) {
     uint32_t tot = np;
 #pragma unroll

@@ -61,3 +61,26 @@ def test_infinite_features_stay_in_their_columns():
         w["norm"][0] = 1e37
     got, want = _frame(change, velocity=100.0)
     _check_columns(got, want, so.OFF_W1, so.OFF_W2, so.FEAT, [2, 3])
+
+
+def test_infinite_pair_sums_stay_in_their_columns():
+    # hidden unit K is 3e38 (q - 1/2), q = 1 - r/h: its sum overflows in the crowd and is 0 in the lattice
+    def change(w):
+        w["W1"][K] = 0.0
+        w["W1"][K, 8:10] = -1.5e38, 3e38
+    got, want = _frame(change)
+    _check_columns(got, want, so.OFF_W2, so.OFF_B2, so.HID, [K])
+    _check_columns(got, want, so.OFF_W1, so.OFF_W2, so.FEAT, [])
+
+
+def test_infinite_messages_stay_in_their_columns():
+    # message A is 1e38 H_K, infinite in the crowd and 0 in the lattice, and no output of W3 uses it (0 times infinity)
+    def change(w):
+        w["W1"][K] = 0.0
+        w["W1"][K, 8:10] = -5.0, 10.0
+        w["W2"][A] = 0.0
+        w["W2"][A, K] = 1e38
+        w["W3"][:, A] = 0.0
+    got, want = _frame(change)
+    _check_columns(got, want, so.OFF_W3, so.OFF_B3, so.HID, [A])
+    _check_columns(got, want, so.OFF_W2, so.OFF_B2, so.HID, [])
