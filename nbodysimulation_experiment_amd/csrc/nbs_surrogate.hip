@@ -44,15 +44,6 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
 }
 __device__ __forceinline__ uint16_t f2bf(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
-__device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
-__device__ __forceinline__ bf16x4 words_to_bf4(uint32_t w0, uint32_t w1) {
-  bf16x4 v;
-  v[0] = (short)(w0 & 0xffffu);
-  v[1] = (short)(w0 >> 16);
-  v[2] = (short)(w1 & 0xffffu);
-  v[3] = (short)(w1 >> 16);
-  return v;
-}
 
 __device__ __forceinline__ floatx16 mfma(bf16x4 a, bf16x4 b, floatx16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, c, 0, 0, 0);
@@ -63,14 +54,6 @@ __device__ __forceinline__ floatx16 zero16() {
 #pragma unroll
   for (int k = 0; k < 16; ++k) z[k] = 0.0f;
   return z;
-}
-
-// B operand of a row-major BF16 weight matrix W (rows = outputs, K inputs):
-// B[k][n] = W[n0 + n][k0 + k].
-__device__ __forceinline__ bf16x4 load_wb(const uint16_t *W, int K, int n0, int k0) {
-  const int c = threadIdx.x & 31, g = (threadIdx.x >> 5) & 1;
-  const uint2 w = *reinterpret_cast<const uint2 *>(W + (size_t)(n0 + c) * K + k0 + 4 * g);
-  return words_to_bf4(w.x, w.y);
 }
 
 // relu(z) as an integer maximum of the bit pattern with 0: negative values
