@@ -146,7 +146,11 @@ class PinnedBuffer {
     return *m;
   }
   static std::vector<uint8_t *> &idle() {
-    static std::vector<uint8_t *> *v = new std::vector<uint8_t *>;
+    static std::vector<uint8_t *> *v = [] {
+      auto *p = new std::vector<uint8_t *>;
+      p->reserve(kPinnedKept);  // giving a buffer back (a destructor) allocates nothing
+      return p;
+    }();
     return *v;
   }
   uint8_t *p_ = nullptr;
