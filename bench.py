@@ -19,8 +19,10 @@ Protocol (inputs resident in HBM in every timed region):
 roofline: the dominant kernel group's limiter.  Its wave64 VALU instructions
 per launch (the rocprofv3 SQ_INSTS_VALU summary of this command in
 profiles/valu_issue.json) over its average launch duration, measured here with
-HIP events on the library's stream, against the VALU issue ceiling of 256 CUs
-x 2.4 GHz x one instruction per CU per cycle; the HBM figure (algorithmic
+HIP events on the library's stream, against a nominal VALU issue rate of 256 CUs
+x 2.4 GHz x one instruction per CU per cycle (FP32 multiplies and additions from
+vector registers reach 1.46 of it, compares 0.9, transcendentals 0.5, so that a
+fraction near 1 tells how busy the VALU is, not how far its limit); the HBM figure (algorithmic
 bytes per launch over the same duration, against 8 TB/s) follows as the
 secondary bound.
 
@@ -53,14 +55,19 @@ sys.path.insert(0, ROOT)
 
 METRIC = "particle-steps/s @1M particles: plain vs surrogate at ≤1% density error"
 HBM_PEAK_GBS = 8000.0
-# MI355X: 256 CUs at 2.4 GHz; a CU issues at most one wave64 VALU instruction
-# per cycle (4 SIMD16 units, 4 cycles each).
+# MI355X: 256 CUs at 2.4 GHz, nominally one wave64 VALU instruction per CU and
+# cycle (4 SIMD16 units, 4 cycles each).  Measured per class: FP32 multiplies
+# from vector registers 894 G/s (1.46 of this rate), with a scalar operand 565,
+# compares and selects 0.9 of it, transcendentals 0.5.
 VALU_PEAK_GINST = 256 * 2.4
 DT = 0.005
 
 # Algorithmic bytes per particle of each kernel group: every particle record
 # crosses HBM once per phase, neighbour re-reads are on-chip.
 #   viscosity_predict: R x,v (16) + W xpred (8) + W key, fill (8) + R key (4)  = 36
+#     (the phase's records; the kernel itself writes no fill: 32 on placed steps,
+#     whose grid group moves 48, and on the others k_count_fill, in the grid
+#     group, writes it)
 #   grid:              R key, fill (8) + W slot, id (8) + R slot, id (8)
 #                      + R xpred, x (16) + W x, prev, id, key (24)              = 64
 #   density:           R x, key (12) + W density, pressure (16)                = 28

@@ -106,9 +106,10 @@ __device__ __forceinline__ void pair_length(float r2, float &r, float &inv) {
 }
 
 // The same results for r2 == 0 or r2 >= 2^-96 (wave_near checks this once per
-// wave), from one v_rsq_f32: y = rsq(x), s0 = x*y, r = s0 + (x - s0^2) * y/2,
-// which is the correctly rounded root for every mantissa, and the reciprocal's
-// Newton step from v_rcp_f32(r) (starting it from y misses the two operands
+// wave), from one v_rsq_f32: y = rsq(x), s0 = x*y, r = s0 + (x - s0^2) * y/2, a
+// Newton step with its residual by FMA (Markstein, as rcp_near), which is the
+// correctly rounded root for every mantissa, and the reciprocal's Newton step
+// from v_rcp_f32(r) (starting it from y misses the two operands
 // whose root has an all-ones mantissa).  x = r2 + 2^-126 is r2 unless r2 == 0,
 // whose r is then 2^-63: 1 - r/h still rounds to 1 for h > 2^-36, and a zero
 // difference times the finite inv is the zero normal.  9 issue cycles against
@@ -486,8 +487,8 @@ __device__ __forceinline__ void plan_tile(const uint32_t *start, const DevScene 
 // and rows read after the tile took five.  A slot range within one scene reads
 // that scene once.  96 scenes, 1.76 M particles: viscosity 66.6 -> 62.5 us,
 // density 45.2 -> 41.9, delta 61.5 -> 60; one scene of 1,048,576: unchanged
-// (its kernels are bound by the walk's issue: of 38.5 us viscosity, 17 remain
-// without the walk, 25 with the walk's tests alone).
+// (of its 38.5 us viscosity, 17 remain without the walk, whose bytes take 8,
+// and 25 with the walk's tests alone).
 template <bool MULTI, int CAP, int SLOTS>
 __device__ __forceinline__ void open_block(const Buffers &b, const DevScene &s0, const uint32_t *start, int i0,
                                            int end, uint32_t key, DevScene &sc, TilePlan &plan, int &cx, int &cy,

@@ -943,10 +943,9 @@ __global__ __launch_bounds__(kSmallGridBlock) void k_scan_small(Buffers b, uint3
 // LDS and leaves the cell starts there, and each particle is then bucketed at
 // its cell start + arrival index: its source slot in tmpSlot, and in binRec
 // the record (source slot, key, cell start, cell end) the rank pass starts
-// from.  Used after the wide viscosity kernel (which leaves the counting to a
-// later kernel) for steps of at most kSmallCountParticles particles: one
-// launch instead of k_count_fill + k_scan_small + k_scatter, and no global
-// atomics.
+// from.  Used for steps of at most kSmallCountParticles particles on small
+// grids, whichever viscosity kernel ran: one launch instead of k_count_fill +
+// k_scan_small + k_scatter, and no global atomics.
 constexpr int kSmallItems = kSmallCountParticles / kSmallGridBlock;  // particles per thread, at most
 __global__ __launch_bounds__(kSmallGridBlock) void k_count_scan_small(Buffers b, int n, uint32_t cells) {
   __shared__ uint32_t hist[kSmallHistWords];  // counts, then cell starts [0, cells], at lds_cell(c)

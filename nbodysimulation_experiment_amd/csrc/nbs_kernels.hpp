@@ -133,9 +133,11 @@ uint32_t launch_grid(const Buffers &b, const DevScene &s0, uint32_t cells, int n
 // one-workgroup scan, every particle binned by the last step, and enough
 // particles for its 1,024-slot workgroups to fill the chip.  Two launches and
 // the counts' reread against k_place's ranking by one workgroup per 1,024
-// slots, whole step: 1,048,576 particles 122.4 us placed and 127.0 not;
-// 262,144: 59.3 and 55.1 (collapsed 826 and 795); 65,536: 41.6 and 42.4
-// (collapsed 703 and 671).
+// slots, whole step at the 0.5h lattice, placed and sorted: 262,144 particles
+// 50.4 and 48.9 us, 394,384 59.6 and 60.5, 524,176 68.8 and 70.1, 784,996 91.7
+// and 94.5, 1,048,576 111.8 and 115.0.  In crowded states sorting is the faster
+// at every one of these sizes (600 steps on: 304 and 288, 300 and 286, 333 and
+// 319, 338 and 328, 354 and 344), which the rule, in n alone, does not see.
 constexpr uint64_t kPlaceMinParticles = 393216;
 bool place_binning(uint64_t n, uint32_t cells, bool allBinned);
 void launch_density(const Buffers &b, const DevParams &p, const DevScene &s0, int n, int cap, hipStream_t stream);

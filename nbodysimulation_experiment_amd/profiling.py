@@ -132,8 +132,8 @@ CUS = 256  # MI355X compute units; GRBM_GUI_ACTIVE is summed over its 8 XCDs
 
 def valu_issue(c: dict, workload: str, steps: int = 0) -> dict:
     """VALU issue utilisation of each kernel group from a counters() result:
-    SQ_INSTS_VALU / (CUS * GRBM_GUI_ACTIVE / 8), a CU issuing at most one wave64
-    VALU instruction per cycle; the single-scene LDS-tile variants pooled by
+    SQ_INSTS_VALU / (CUS * GRBM_GUI_ACTIVE / 8), nominally one wave64 VALU
+    instruction per CU and cycle; the single-scene LDS-tile variants pooled by
     dispatches (multi-scene variants, "<t,N>", belong to other workloads).
     Also the wave64 VALU instructions per launch of each group (summed over
     the group's kernels), which bench.py divides by its measured launch
